@@ -17,11 +17,14 @@
 // (region, rank) are taken from a queue in order, with every rank of a team
 // queued consecutively, by a grid that is co-resident on the device.
 //
-// Work layout inside a chunk: a quad of 4 lanes evaluates one sample; lane q
-// of the quad owns mixture components k = 4j + q (j < 8), so a wave evaluates
-// 16 samples x 32 components per step with the component parameters held in
-// registers.  The per-sample pdf is a 2-step quad reduction; per-lane sums over
-// the chunk are reduced over quads (xor-shuffles) and waves (fixed order).
+// Work layout inside a chunk: lane q of a quad of 4 lanes owns mixture
+// components k = 4j + q (j < 8), their parameters held in registers, and a
+// quad evaluates four samples per step (one per lane for everything that is
+// per sample), so a wave evaluates 64 samples x 32 components per step.  The
+// contractions - the dot products of samples with component directions and
+// the sums over samples of responsibility times sample - run on the matrix
+// cores (see the sample passes).  Per-lane sums over the chunk are reduced
+// over quads and waves (fixed order).
 // Per-component M-step / split / merge logic runs in wave 0 with one lane per
 // component, serial decisions in lane 0.  The mean-cosine -> kappa inversion
 // and the log-likelihood convergence test are evaluated in FP64; everything
@@ -97,14 +100,16 @@ struct Shared {
   SuffStats cur;
   SuffStats tmp;
   SplitStatsState lsplit;
-  float red[RWAVES][32][8];
+  float red[RWAVES][6][32];  // sample pass: per-wave sums of the chunk (field, component)
+  alignas(16) float comp[32][8];   // sample pass: direction, kappa log2(e) and weight times norm of each component
   alignas(16) float frame[32][8];  // split statistics: tangent frame of each component (x axis, y axis, 2 unused)
   float cost[32 * 32];
   float selfp[32][6];      // merging: product of each component with itself (direction, kappa, norm, scale)
   float term[64][3];       // merging: the three cost terms of up to 64 pairs
   float pre[10];           // merging: weight, direction and mean cosine of the chosen pair before the merge
   float scal[RWAVES][8];
-  float stage[5][kChunk];  // sample pass: the current chunk's dx, dy, dz, w and pdf or distance
+  alignas(16) float stage[5][kChunk];  // sample pass: the current chunk's dx, dy, dz, w and pdf or distance,
+                                       // at stage_pos() of the sample's place in the chunk
   uint32_t stageKey;       // first sample (absolute index) of the chunk held in stage[0..3], ~0: none
   uint32_t stageCnt;       // its samples
   const float* stageExtra; // the array whose values stage[4] holds for that chunk (null: none)
@@ -195,31 +200,34 @@ __device__ __forceinline__ void split_zero_slot(SplitStatsState& s, int k) {
 __device__ __forceinline__ int vec_lim(int W, int K) { int l = ((K + W - 1) / W) * W; return l > 32 ? 32 : l; }
 
 // ------------------------------------------------------------ sample passes
-// Loads this lane's component parameters (k = 4j + q) into registers.
-struct CompRegs {
-  float x[8], y[8], z[8], kap2[8], wn[8];  // kap2 = kappa log2(e)
-};
-
-__device__ __forceinline__ void load_comps(const VMMParams& V, int q, CompRegs& c) {
-  const int K = V.K;
-#pragma unroll
-  for (int j = 0; j < 8; j++) {
-    const int k = 4 * j + q;
-    const bool a = k < K;
-    c.x[j] = a ? V.mux[k] : 0.f;
-    c.y[j] = a ? V.muy[k] : 0.f;
-    c.z[j] = a ? V.muz[k] : 1.f;
-    c.kap2[j] = a ? V.kappa[k] * 1.44269504088896341f : 0.f;
-    c.wn[j] = a ? V.w[k] * V.norm[k] : 0.f;
+// Component parameters of a pass, as the sample loops read them: one row per
+// component (zero weight from K on).  Callers synchronise before reading.
+__device__ __forceinline__ void fill_comps(Shared& sh) {
+  const VMMParams& V = sh.S.vmm;
+  if (threadIdx.x < 32) {
+    const int k = threadIdx.x;
+    const bool a = k < V.K;
+    float* c = sh.comp[k];
+    c[0] = a ? V.mux[k] : 0.f;
+    c[1] = a ? V.muy[k] : 0.f;
+    c[2] = a ? V.muz[k] : 1.f;
+    c[3] = a ? V.kappa[k] * 1.44269504088896341f : 0.f;  // kappa log2(e)
+    c[4] = a ? V.w[k] * V.norm[k] : 0.f;
   }
 }
 
-// sum over the 4 lanes of a quad (DPP quad permutes: lane ^ 1, then lane ^ 2);
-// every lane of the quad gets the same bits, as IEEE addition commutes
-__device__ __forceinline__ float quad_sum(float v) {
-  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));
-  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xF, 0xF, true));
-  return v;
+// This lane's components (k = 4j + q).
+struct CompRegs {
+  float x[8], y[8], z[8], kap2[8], wn[8];
+};
+
+__device__ __forceinline__ void load_comp(const Shared& sh, int q, int j, CompRegs& c) {
+  const float4 v = *reinterpret_cast<const float4*>(&sh.comp[4 * j + q][0]);
+  c.x[j] = v.x;
+  c.y[j] = v.y;
+  c.z[j] = v.z;
+  c.kap2[j] = v.w;
+  c.wn[j] = sh.comp[4 * j + q][4];
 }
 
 // Calls f with std::integral_constant<int, JT> for the smallest even JT >= J
@@ -234,39 +242,67 @@ __device__ __forceinline__ void with_groups(int J, F&& f) {
   else f(std::integral_constant<int, 2>());
 }
 
-// soft_eval for the first JT component groups of this lane (e[j] = 0 for
-// j >= JT), with no branch between the components
-template <int JT>
-__device__ __forceinline__ float soft_eval_t(const CompRegs& c, float dx, float dy, float dz, float e[8]) {
-  float part = 0.f;
-#pragma unroll
-  for (int j = 0; j < 8; j++) {
-    if (j < JT) {
-      const float ct = dot3f(dx, dy, dz, c.x[j], c.y[j], c.z[j]);
-      e[j] = c.wn[j] * __builtin_amdgcn_exp2f(fminf(fmaf(c.kap2[j], ct, -c.kap2[j]), 0.f));
-      part += e[j];
-    } else {
-      e[j] = 0.f;
-    }
-  }
-  return quad_sum(part);
+// Matrix-core form of a quad's work.  v_mfma_f32_4x4x1_16b_f32 works on 16
+// independent 4 x 4 blocks, and block b is lanes 4b .. 4b + 3: D[i][l] = A[i] *
+// B[l] + C[i][l] with A[i] and B[l] one register of lanes i and l and row i of
+// C and D the i-th of four registers.  A block is a quad, every element is one
+// fused multiply-add rounded once (bit for bit fmaf, denormals and NaN payloads
+// included), so
+//   * with A the lanes' own samples and B the lanes' components, three of them
+//     give the dot products of four samples with four components;
+//   * with A the lanes' features of one sample and B the lanes' responsibilities
+//     for it, one adds that sample to four sums of four components,
+// in the same operations and order as one sample after the other.  The
+// instruction holds the matrix core for 8 cycles where its fused
+// multiply-adds take 16 on the vector unit, which goes on with the
+// exponentials meanwhile.
+typedef float Mat4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ Mat4 quad_mfma(float a, float b, Mat4 c) {
+  return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 0, 0, 0);
 }
 
-// e_k = w_k norm_k exp(kappa_k min(mu_k.d - 1, 0)), evaluated as
-// w_k norm_k 2^min(kap2_k mu_k.d - kap2_k, 0); returns the quad-wide pdf
-__device__ __forceinline__ float soft_eval(const CompRegs& c, int J, float dx, float dy, float dz, float e[8]) {
-  float part = 0.f;
+// value of quad lane L in all four lanes
+template <int L>
+__device__ __forceinline__ float quad_bcast(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), L * 0x55, 0xF, 0xF, true));
+}
+
+// Lane i of a quad gets the sum over the quad of v[i], added as
+// (v@i + v@(i ^ 1)) + (v@(i ^ 2) + v@(i ^ 3)).
+__device__ __forceinline__ float quad_sum_own(int q, const float v[4]) {
+  const bool odd = (q & 1) != 0, hi = (q & 2) != 0;
+  const float k0 = odd ? v[1] : v[0], s0 = odd ? v[0] : v[1];
+  const float k1 = odd ? v[3] : v[2], s1 = odd ? v[2] : v[3];
+  const float t0 = k0 + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(s0), 0xB1, 0xF, 0xF, true));
+  const float t1 = k1 + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(s1), 0xB1, 0xF, 0xF, true));
+  const float k2 = hi ? t1 : t0, s2 = hi ? t0 : t1;
+  return k2 + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(s2), 0x4E, 0xF, 0xF, true));
+}
+
+// e[j][i] = w_k norm_k exp(kappa_k min(mu_k.d_i - 1, 0)) of this lane's
+// component k = 4j + q for the quad's sample i (the sample whose direction is
+// x, y, z in lane i), evaluated as w_k norm_k 2^min(kap2_k mu_k.d - kap2_k, 0),
+// with no branch between the components; returns the pdf of the lane's own
+// sample.
+template <int JT>
+__device__ __forceinline__ float soft_eval_quad(const CompRegs& c, int q, float x, float y, float z, Mat4 e[8]) {
+  float part[4] = {0.f, 0.f, 0.f, 0.f};
+  const Mat4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int j = 0; j < 8; j++) {
-    if (j < J) {
-      const float ct = dot3f(dx, dy, dz, c.x[j], c.y[j], c.z[j]);
-      e[j] = c.wn[j] * __builtin_amdgcn_exp2f(fminf(fmaf(c.kap2[j], ct, -c.kap2[j]), 0.f));
-      part += e[j];
-    } else {
-      e[j] = 0.f;
+  for (int j = 0; j < JT; j++) e[j] = quad_mfma(z, c.z[j], zero);
+#pragma unroll
+  for (int j = 0; j < JT; j++) e[j] = quad_mfma(y, c.y[j], e[j]);
+#pragma unroll
+  for (int j = 0; j < JT; j++) e[j] = quad_mfma(x, c.x[j], e[j]);
+#pragma unroll
+  for (int j = 0; j < JT; j++) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      e[j][i] = c.wn[j] * __builtin_amdgcn_exp2f(fminf(fmaf(c.kap2[j], e[j][i], -c.kap2[j]), 0.f));
+      part[i] += e[j][i];
     }
   }
-  return quad_sum(part);
+  return quad_sum_own(q, part);
 }
 
 // Cross-lane sums without LDS traffic: DPP row rotations inside each row of
@@ -283,12 +319,32 @@ __device__ __forceinline__ float cross_row_sum(float v) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
-// sum over the 16 lanes of a wave with the same lane % 4 (the quads' lane q);
-// lanes 0..3 hold the sums of q = 0..3
-__device__ __forceinline__ float quad_group_sum(float v) {
-  v += PGL_ROW_ROR(v, 4);
-  v += PGL_ROW_ROR(v, 8);
-  return cross_row_sum(v);
+// Sums over the 16 quads of a wave, for eight values of every lane at once.
+// One value's sum is ((v0 + v3) + (v2 + v1)) over the four quads of each row
+// of 16 lanes, then (r0 + r1) + (r2 + r3) over the rows.  Every stage halves
+// the registers it works on instead of leaving idle lanes: two values share
+// the even and odd quads, two such pairs the even and odd rows, two of those
+// the halves of the wave: 22 instructions for eight values where eight sums
+// of their own take 64, and one store (ending a chunk of the E-step, 37 sums
+// of their own, took 3.0 us with two workgroups on the CU, more than its
+// samples).  Lane l ends with the sum, over the lanes of its l % 4, of value
+// sum8_index(l).
+__device__ __forceinline__ int sum8_index(int lane) { return ((lane >> 5) << 2) | ((lane >> 3) & 2) | ((lane >> 2) & 1); }
+__device__ __forceinline__ float quad_pair_sum(bool odd, float a, float b) {
+  const float bs = PGL_ROW_ROR(b, 4);  // the previous quad's b
+  const float m = odd ? bs : a, n = odd ? a : bs;
+  const float t = m + PGL_ROW_ROR(n, 4);
+  return t + PGL_ROW_ROR(t, 8);
+}
+__device__ __forceinline__ float sum8(bool odd, float v0, float v1, float v2, float v3, float v4, float v5, float v6,
+                                      float v7) {
+  const float p0 = quad_pair_sum(odd, v0, v1), p1 = quad_pair_sum(odd, v2, v3);
+  const float p2 = quad_pair_sum(odd, v4, v5), p3 = quad_pair_sum(odd, v6, v7);
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(p0), __float_as_uint(p1), false, false);
+  const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(p2), __float_as_uint(p3), false, false);
+  const float u = __uint_as_float(a[0]) + __uint_as_float(a[1]), w = __uint_as_float(b[0]) + __uint_as_float(b[1]);
+  const auto c = __builtin_amdgcn_permlane32_swap(__float_as_uint(u), __float_as_uint(w), false, false);
+  return __uint_as_float(c[0]) + __uint_as_float(c[1]);
 }
 
 // sum over the 64 lanes of a wave, valid in lane 0
@@ -308,11 +364,13 @@ __device__ __forceinline__ void kfold(float& sum, float& comp, float x) {
   sum = t;
 }
 
-// value v of the current chunk from the per-wave partials (fixed order)
-__device__ __forceinline__ float chunk_value(const Shared& sh, int v, int F, int NS) {
+// value v of the current chunk from the per-wave partials (fixed order);
+// components from KG on have none (zero)
+__device__ __forceinline__ float chunk_value(const Shared& sh, int v, int F, int NS, int KG) {
   if (v < 32 * F) {
     const int f = v >> 5, k = v & 31;
-    return (sh.red[0][k][f] + sh.red[1][k][f]) + (sh.red[2][k][f] + sh.red[3][k][f]);
+    if (k >= KG) return 0.f;
+    return (sh.red[0][f][k] + sh.red[1][f][k]) + (sh.red[2][f][k] + sh.red[3][f][k]);
   }
   if (v >= kScal && v < kScal + NS) {
     const int i = v - kScal;
@@ -358,10 +416,12 @@ __device__ void team_barrier(Shared& sh, Team& tm) {
 
 // End of a chunk: value v = threadIdx.x of chunk c goes into the running fold
 // (T = 1, chunks arrive in order) or to the team's partial buffer.
-__device__ __forceinline__ void chunk_out(const Shared& sh, const Team& tm, uint32_t c, int F, int NS, int llIdx,
-                                          float& fs, float& fc, double& fd) {
+// The next chunk's sums are written behind the barrier after its staging, so
+// no barrier is needed here.
+__device__ __forceinline__ void chunk_out(const Shared& sh, const Team& tm, uint32_t c, int F, int NS, int KG,
+                                          int llIdx, float& fs, float& fc, double& fd) {
   const int v = threadIdx.x;
-  const float x = chunk_value(sh, v, F, NS);
+  const float x = chunk_value(sh, v, F, NS, KG);
   if (tm.T == 1) {
     if (v == llIdx) fd += (double)x;
     else kfold(fs, fc, x);
@@ -402,8 +462,19 @@ __device__ void pass_finish(Shared& sh, Team& tm, int llIdx, float fs, float fc,
   __syncthreads();
 }
 
+// Place of sample o of a chunk in the staging arrays: quad p of the workgroup
+// takes samples p, p + 64, p + 128, ... in that order, four per step, and
+// finds the four of a step next to each other, so that a lane reads its own
+// sample without bank conflicts and the quad's four values of one array are
+// one 16-byte read.
+__device__ __forceinline__ uint32_t stage_pos(uint32_t o) {
+  return (o & ~255u) | ((o & 63u) << 2) | ((o >> 6) & 3u);
+}
+
 // Copies samples [first, first + cnt) of the region's stream into the
-// staging arrays (dx, dy, dz, w, and pdf or distance when extra is set):
+// staging arrays (dx, dy, dz, w, and pdf or distance when extra is set),
+// followed up to the end of the last step by samples that add zero to every
+// sum (direction and weight 0, pdf or distance 1):
 // every thread issues all of its coalesced loads at once, so a chunk costs
 // one memory latency instead of one per sample step.  A chunk already
 // staged (every pass reads the same samples, and a rank takes the same
@@ -413,6 +484,7 @@ __device__ void pass_finish(Shared& sh, Team& tm, int llIdx, float fs, float fc,
 __device__ __forceinline__ void stage_chunk(Shared& sh, const RegionSamples& rs, uint32_t first, uint32_t cnt,
                                             const float* __restrict__ extra) {
   const int tid = threadIdx.x;
+  const uint32_t padded = (cnt + RT - 1) / RT * RT;
   const bool have = sh.stageKey == first && sh.stageCnt == cnt;
   const bool loadMain = !have;
   const bool loadExtra = extra != nullptr && !(have && sh.stageExtra == extra);
@@ -421,6 +493,8 @@ __device__ __forceinline__ void stage_chunk(Shared& sh, const RegionSamples& rs,
 #pragma unroll
   for (int m = 0; m < (int)(kChunk / RT); m++) {
     const uint32_t o = tid + m * RT;
+#pragma unroll
+    for (int a = 0; a < 5; a++) v[m][a] = a < 4 ? 0.f : 1.f;
     if (o < cnt) {
       const uint32_t i = first + o;
       if (loadMain) {
@@ -435,12 +509,13 @@ __device__ __forceinline__ void stage_chunk(Shared& sh, const RegionSamples& rs,
 #pragma unroll
   for (int m = 0; m < (int)(kChunk / RT); m++) {
     const uint32_t o = tid + m * RT;
-    if (o < cnt) {
+    if (o < padded) {
+      const uint32_t p = stage_pos(o);
       if (loadMain) {
 #pragma unroll
-        for (int a = 0; a < 4; a++) sh.stage[a][o] = v[m][a];
+        for (int a = 0; a < 4; a++) sh.stage[a][p] = v[m][a];
       }
-      if (loadExtra) sh.stage[4][o] = v[m][4];
+      if (loadExtra) sh.stage[4][p] = v[m][4];
     }
   }
 }
@@ -475,68 +550,74 @@ __device__ __forceinline__ RankChunks rank_chunks(const Shared& sh, const Team& 
   return r;
 }
 
-// Per-lane E-step sums of a chunk.
+// Per-lane E-step sums of a chunk: b[j] holds sum of gamma w (dx, dy, dz, 1)
+// of component 4j + q; the log-likelihood and the unassigned sums are the
+// quad's in every lane.
 struct EStepAcc {
-  float* bx;
-  float* by;
-  float* bz;
-  float* bw;
-  float& ll;
-  float& u0;
-  float& u1;
-  float& u2;
-  float& u3;
+  Mat4 b[8];
+  float ll, u0, u1, u2, u3;
 };
 
-// One sample of the E-step, without branches: a sample the mixture does not
-// cover (pdf <= 1e-16) adds zero to the component sums and its weight to the
-// unassigned sums (lane q = 0 of the quad, like the log-likelihood).  e and
-// pdf come from soft_eval_t.
-template <int JT>
-__device__ __forceinline__ void estep_accumulate(int q, float dx, float dy, float dz, float w, const float e[8],
-                                                 float pdf, EStepAcc& a) {
-  const bool ok = pdf > 1e-16f;
-  const float wu = (!ok && q == 0) ? w : 0.f;
-  a.u0 += wu;
-  a.u1 = fmaf(dx, wu, a.u1);
-  a.u2 = fmaf(dy, wu, a.u2);
-  a.u3 = fmaf(dz, wu, a.u3);
-  const float lp = fmaf(w, logf(pdf), a.ll);
-  a.ll = (ok && q == 0) ? lp : a.ll;
-  const float r = ok ? w * __builtin_amdgcn_rcpf(pdf) : 0.f;
-  const float rx = r * dx, ry = r * dy, rz = r * dz;
-#pragma unroll
-  for (int j = 0; j < JT; j++) {
-    a.bx[j] = fmaf(e[j], rx, a.bx[j]);
-    a.by[j] = fmaf(e[j], ry, a.by[j]);
-    a.bz[j] = fmaf(e[j], rz, a.bz[j]);
-    a.bw[j] = fmaf(e[j], r, a.bw[j]);
-  }
+// The quad's sample i of the unassigned sums.
+template <int L>
+__device__ __forceinline__ void estep_unassigned(EStepAcc& a, float x, float y, float z, float wu) {
+  const float w = quad_bcast<L>(wu);
+  a.u0 += w;
+  a.u1 = fmaf(quad_bcast<L>(x), w, a.u1);
+  a.u2 = fmaf(quad_bcast<L>(y), w, a.u2);
+  a.u3 = fmaf(quad_bcast<L>(z), w, a.u3);
 }
 
-// The staged chunk's samples s = quad, quad + 64, ... in that order.  Two
-// samples per step: both are evaluated before either is accumulated, so the
-// two exp/dot chains overlap; the sums still take the samples one after the
-// other, in sample order.
+// The staged chunk's samples, four per quad and step.  Every sum takes the
+// quad's samples in sample order.  A sample the mixture does not cover (pdf <=
+// 1e-16) adds zero to the component sums and its weight to the unassigned
+// sums.
+//
+// Bound by the vector unit: per step a lane evaluates 4 JT exponentials, each
+// with a fused multiply-add, a minimum, a product and an addition beside it;
+// what is per sample (logarithm, reciprocal) is done by one lane per sample,
+// and the 7 JT multiply-accumulate groups are matrix instructions: 319
+// instructions per 64 samples and 32 components, 1110 with the dot products
+// and sums on the vector unit and every lane of a quad on the same sample.
+// With the chunk sums below, a first update of 8 M samples (363 regions) takes
+// 6.3 instead of 9.4 ms in the region kernel, the next one 2.4 instead of 3.2,
+// bit for bit the same.
 template <int JT>
-__device__ __forceinline__ void estep_chunk(const Shared& sh, const CompRegs& c, int q, int quad, uint32_t cnt,
-                                            EStepAcc& a) {
-  uint32_t s = quad;
-  for (; s + RT / 4 < cnt; s += RT / 2) {
-    const uint32_t t = s + RT / 4;
-    const float ax = sh.stage[0][s], ay = sh.stage[1][s], az = sh.stage[2][s], aw = sh.stage[3][s];
-    const float bx = sh.stage[0][t], by = sh.stage[1][t], bz = sh.stage[2][t], bw = sh.stage[3][t];
-    float ea[8], eb[8];
-    const float pa = soft_eval_t<JT>(c, ax, ay, az, ea);
-    const float pb = soft_eval_t<JT>(c, bx, by, bz, eb);
-    estep_accumulate<JT>(q, ax, ay, az, aw, ea, pa, a);
-    estep_accumulate<JT>(q, bx, by, bz, bw, eb, pb, a);
-  }
-  if (s < cnt) {
-    const float ax = sh.stage[0][s], ay = sh.stage[1][s], az = sh.stage[2][s], aw = sh.stage[3][s];
-    float ea[8];
-    const float pa = soft_eval_t<JT>(c, ax, ay, az, ea);
-    estep_accumulate<JT>(q, ax, ay, az, aw, ea, pa, a);
+__device__ __forceinline__ void estep_chunk(const Shared& sh, const CompRegs& c, int q, uint32_t cnt, EStepAcc& a) {
+  const uint32_t tid = threadIdx.x;
+  for (uint32_t s0 = 0; s0 < cnt; s0 += RT) {
+    const float x = sh.stage[0][s0 + tid], y = sh.stage[1][s0 + tid], z = sh.stage[2][s0 + tid];
+    const float w = sh.stage[3][s0 + tid];
+    // this lane's feature (dx, dy, dz or 1) of the quad's four samples
+    const float4 row = *reinterpret_cast<const float4*>(&sh.stage[q][s0 + (tid & ~3u)]);
+    const bool one = q == 3;
+    const float g0 = one ? 1.f : row.x, g1 = one ? 1.f : row.y, g2 = one ? 1.f : row.z, g3 = one ? 1.f : row.w;
+    Mat4 e[8];
+    const float pdf = soft_eval_quad<JT>(c, q, x, y, z, e);
+    const bool ok = pdf > 1e-16f;
+    const float lw = ok ? w : 0.f, lp = ok ? logf(pdf) : 0.f;
+    const float r = ok ? w * __builtin_amdgcn_rcpf(pdf) : 0.f;
+    a.ll = fmaf(quad_bcast<0>(lw), quad_bcast<0>(lp), a.ll);
+    a.ll = fmaf(quad_bcast<1>(lw), quad_bcast<1>(lp), a.ll);
+    a.ll = fmaf(quad_bcast<2>(lw), quad_bcast<2>(lp), a.ll);
+    a.ll = fmaf(quad_bcast<3>(lw), quad_bcast<3>(lp), a.ll);
+    if (__ballot(!ok)) {
+      const float wu = ok ? 0.f : w;
+      estep_unassigned<0>(a, x, y, z, wu);
+      estep_unassigned<1>(a, x, y, z, wu);
+      estep_unassigned<2>(a, x, y, z, wu);
+      estep_unassigned<3>(a, x, y, z, wu);
+    }
+    const float f0 = quad_bcast<0>(r) * g0, f1 = quad_bcast<1>(r) * g1, f2 = quad_bcast<2>(r) * g2,
+                f3 = quad_bcast<3>(r) * g3;
+#pragma unroll
+    for (int j = 0; j < JT; j++) a.b[j] = quad_mfma(f0, e[j][0], a.b[j]);
+#pragma unroll
+    for (int j = 0; j < JT; j++) a.b[j] = quad_mfma(f1, e[j][1], a.b[j]);
+#pragma unroll
+    for (int j = 0; j < JT; j++) a.b[j] = quad_mfma(f2, e[j][2], a.b[j]);
+#pragma unroll
+    for (int j = 0; j < JT; j++) a.b[j] = quad_mfma(f3, e[j][3], a.b[j]);
   }
 }
 
@@ -545,12 +626,17 @@ __device__ __forceinline__ void estep_chunk(const Shared& sh, const CompRegs& c,
 // fin[kScal+0..3] = unassigned (w, w dx, w dy, w dz).
 __device__ void pass_estep(Shared& sh, Team& tm, const RegionSamples& rs, uint32_t base, uint32_t n) {
   const unsigned long long tPass = wall_clock64();
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = tid & 3, quad = tid >> 2;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = tid & 3;
   const VMMParams& V = sh.S.vmm;
   const int K = V.K;
   const int J = (K + 3) >> 2;
+  const int vi = sum8_index(lane);
+  const bool odd = (lane & 4) != 0;
+  fill_comps(sh);
+  __syncthreads();
   CompRegs c;
-  load_comps(V, q, c);
+#pragma unroll
+  for (int j = 0; j < 8; j++) load_comp(sh, q, j, c);
   float fs = 0.f, fc = 0.f;
   double fd = 0.0;
   const RankChunks rc = rank_chunks(sh, tm, base);
@@ -560,39 +646,25 @@ __device__ void pass_estep(Shared& sh, Team& tm, const RegionSamples& rs, uint32
     stage_chunk(sh, rs, base + cb, ce - cb, nullptr);
     __syncthreads();
     stage_mark(sh, base + cb, ce - cb, nullptr);
-    float bx[8], by[8], bz[8], bw[8];
+    EStepAcc a;
 #pragma unroll
-    for (int j = 0; j < 8; j++) bx[j] = by[j] = bz[j] = bw[j] = 0.f;
-    float ll = 0.f, u0 = 0.f, u1 = 0.f, u2 = 0.f, u3 = 0.f;
-    EStepAcc a{bx, by, bz, bw, ll, u0, u1, u2, u3};
-    with_groups(J, [&](auto jt) { estep_chunk<decltype(jt)::value>(sh, c, q, quad, ce - cb, a); });
+    for (int j = 0; j < 8; j++) a.b[j] = Mat4{0.f, 0.f, 0.f, 0.f};
+    a.ll = a.u0 = a.u1 = a.u2 = a.u3 = 0.f;
+    with_groups(J, [&](auto jt) {
+      constexpr int JT = decltype(jt)::value;
+      estep_chunk<JT>(sh, c, q, ce - cb, a);
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const float vx = quad_group_sum(bx[j]);
-      const float vy = quad_group_sum(by[j]);
-      const float vz = quad_group_sum(bz[j]);
-      const float vw = quad_group_sum(bw[j]);
-      if (lane < 4) {
-        const int k = 4 * j + lane;
-        sh.red[wave][k][0] = vx;
-        sh.red[wave][k][1] = vy;
-        sh.red[wave][k][2] = vz;
-        sh.red[wave][k][3] = vw;
+      for (int j = 0; j < JT; j += 2) {
+        const Mat4 b0 = a.b[j], b1 = a.b[j + 1];
+        const float s = sum8(odd, b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[3]);
+        if ((lane & 8) == 0) sh.red[wave][vi & 3][4 * (j + (vi >> 2)) + q] = s;
       }
-    }
-    // lanes q != 0 hold zeros for the per-sample scalars
-    const float vll = wave_sum0(ll);
-    const float v0 = wave_sum0(u0), v1 = wave_sum0(u1), v2 = wave_sum0(u2), v3 = wave_sum0(u3);
-    if (lane == 0) {
-      sh.scal[wave][0] = vll;
-      sh.scal[wave][1] = v0;
-      sh.scal[wave][2] = v1;
-      sh.scal[wave][3] = v2;
-      sh.scal[wave][4] = v3;
-    }
+    });
+    // lane q of a quad takes the quad's log-likelihood, w, w dx or w dy; w dz is apart
+    const float sc = cross_row_sum(quad_pair_sum(odd, q == 0 ? a.ll : (q == 1 ? a.u0 : (q == 2 ? a.u1 : a.u2)), a.u3));
+    if (lane < 5) sh.scal[wave][lane] = sc;
     __syncthreads();
-    chunk_out(sh, tm, ch, 4, 5, kScal, fs, fc, fd);
-    __syncthreads();
+    chunk_out(sh, tm, ch, 4, 5, 4 * J, kScal, fs, fc, fd);
   }
   pass_finish(sh, tm, kScal, fs, fc, fd);
   if (tid == 0) {
@@ -606,17 +678,22 @@ __device__ void pass_estep(Shared& sh, Team& tm, const RegionSamples& rs, uint32
 // fin[32+k] = sum of w g_k (g_k pdf / w_k).
 __device__ void pass_distances(Shared& sh, Team& tm, const RegionSamples& rs, uint32_t base, uint32_t n) {
   const unsigned long long tPass = wall_clock64();
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = tid & 3, quad = tid >> 2;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = tid & 3;
   const VMMParams& V = sh.S.vmm;
   const int K = V.K;
   const int J = (K + 3) >> 2;
+  fill_comps(sh);
+  __syncthreads();
   CompRegs c;
-  load_comps(V, q, c);
-  float invw[8];
 #pragma unroll
-  for (int j = 0; j < 8; j++) {
-    const int k = 4 * j + q;
-    invw[j] = k < K ? 1.f / V.w[k] : 0.f;
+  for (int j = 0; j < 8; j++) load_comp(sh, q, j, c);
+  const int vi = sum8_index(lane);
+  const bool odd = (lane & 4) != 0;
+  float invw[2];  // of the components whose sums this lane ends with
+#pragma unroll
+  for (int m = 0; m < 2; m++) {
+    const int k = 4 * (4 * m + (vi >> 1)) + q;
+    invw[m] = k < K ? 1.f / V.w[k] : 0.f;
   }
   float fs = 0.f, fc = 0.f;
   double fd = 0.0;
@@ -627,40 +704,47 @@ __device__ void pass_distances(Shared& sh, Team& tm, const RegionSamples& rs, ui
     stage_chunk(sh, rs, base + cb, ce - cb, rs.dist);
     __syncthreads();
     stage_mark(sh, base + cb, ce - cb, rs.dist);
-    float ad[8], aw[8];
+    Mat4 acc[8];  // rows 0 and 1: the two sums of component 4j + q (rows 2 and 3 repeat row 1)
 #pragma unroll
-    for (int j = 0; j < 8; j++) ad[j] = aw[j] = 0.f;
+    for (int j = 0; j < 8; j++) acc[j] = Mat4{0.f, 0.f, 0.f, 0.f};
     const uint32_t cnt = ce - cb;
     with_groups(J, [&](auto jt) {
       constexpr int JT = decltype(jt)::value;
-      for (uint32_t s = quad; s < cnt; s += RT / 4) {
-        const float dx = sh.stage[0][s], dy = sh.stage[1][s], dz = sh.stage[2][s], w = sh.stage[3][s];
-        float e[8];
-        const float pdf = soft_eval_t<JT>(c, dx, dy, dz, e);
+      for (uint32_t s0 = 0; s0 < cnt; s0 += RT) {
+        const float x = sh.stage[0][s0 + tid], y = sh.stage[1][s0 + tid], z = sh.stage[2][s0 + tid];
+        const float w = sh.stage[3][s0 + tid];
+        Mat4 e[8];
+        const float pdf = soft_eval_quad<JT>(c, q, x, y, z, e);
         const bool ok = pdf > 1e-16f;  // other samples add zero
         // w g_k (g_k pdf / w_k) = (w / pdf) e_k^2 / w_k; 1 / w_k is applied to the chunk sums
+        const float dist = sh.stage[4][s0 + tid];
         const float wip = ok ? w * __builtin_amdgcn_rcpf(pdf) : 0.f;
-        const float wipd = ok ? wip * __builtin_amdgcn_rcpf(sh.stage[4][s]) : 0.f;
+        const float ird = __builtin_amdgcn_rcpf(dist);
+        const float wipd = ok ? wip * ird : 0.f;
+        // broadcast outside the selects: a lane reads lanes that select otherwise
+        const float p0 = quad_bcast<0>(wip), p1 = quad_bcast<1>(wip), p2 = quad_bcast<2>(wip), p3 = quad_bcast<3>(wip);
+        const float d0 = quad_bcast<0>(wipd), d1 = quad_bcast<1>(wipd), d2 = quad_bcast<2>(wipd),
+                    d3 = quad_bcast<3>(wipd);
+        const bool first = q == 0;
+        const float f0 = first ? d0 : p0, f1 = first ? d1 : p1, f2 = first ? d2 : p2, f3 = first ? d3 : p3;
 #pragma unroll
-        for (int j = 0; j < JT; j++) {
-          const float e2 = e[j] * e[j];
-          ad[j] = fmaf(e2, wipd, ad[j]);
-          aw[j] = fmaf(e2, wip, aw[j]);
-        }
+        for (int j = 0; j < JT; j++) acc[j] = quad_mfma(f0, e[j][0] * e[j][0], acc[j]);
+#pragma unroll
+        for (int j = 0; j < JT; j++) acc[j] = quad_mfma(f1, e[j][1] * e[j][1], acc[j]);
+#pragma unroll
+        for (int j = 0; j < JT; j++) acc[j] = quad_mfma(f2, e[j][2] * e[j][2], acc[j]);
+#pragma unroll
+        for (int j = 0; j < JT; j++) acc[j] = quad_mfma(f3, e[j][3] * e[j][3], acc[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < JT; j += 4) {
+        const float s = sum8(odd, acc[j][0], acc[j][1], acc[j + 1][0], acc[j + 1][1], acc[j + 2][0], acc[j + 2][1],
+                             acc[j + 3][0], acc[j + 3][1]);
+        if ((lane & 8) == 0) sh.red[wave][vi & 1][4 * (j + (vi >> 1)) + q] = s * invw[j / 4];
       }
     });
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const float vd = quad_group_sum(ad[j]) * invw[j];
-      const float vw = quad_group_sum(aw[j]) * invw[j];
-      if (lane < 4) {
-        sh.red[wave][4 * j + lane][0] = vd;
-        sh.red[wave][4 * j + lane][1] = vw;
-      }
-    }
     __syncthreads();
-    chunk_out(sh, tm, ch, 2, 0, -1, fs, fc, fd);
-    __syncthreads();
+    chunk_out(sh, tm, ch, 2, 0, 4 * J, -1, fs, fc, fd);
   }
   pass_finish(sh, tm, -1, fs, fc, fd);
   if (tid == 0) { sh.S.auxEvals += (float)n * (float)K; sh.S.prof[3] += (float)(wall_clock64() - tPass); }
@@ -681,14 +765,13 @@ struct SplitAcc {
   float& cnt;
 };
 
-// Split statistics of one sample against component group j (frame f0, f1):
-// vmf = e[j], ip = 1 / pdf, cf = chi-square factor, wip = w / pdf.
-__device__ __forceinline__ void split_add(SplitAcc& a, int j, float4 f0, float2 f1, float dx, float dy, float dz,
-                                          float vmf, float ip, float cf, float wip) {
+// Split statistics of one sample against component group j: vmf = its share
+// of the pdf, lx and ly its coordinates in the component's frame, ip = 1 / pdf,
+// cf = chi-square factor, wip = w / pdf.
+__device__ __forceinline__ void split_add(SplitAcc& a, int j, float lx, float ly, float vmf, float ip, float cf,
+                                          float wip) {
   a.chi[j] += vmf > 0.f ? vmf * cf : 0.f;
   a.sa[j] = fmaf(vmf, ip, a.sa[j]);
-  const float lx = dot3f(f0.x, f0.y, f0.z, dx, dy, dz);
-  const float ly = dot3f(f0.w, f1.x, f1.y, dx, dy, dz);
   const float aw = vmf * wip;
   a.sw[j] += aw;
   a.cx[j] = fmaf(aw, lx * lx, a.cx[j]);
@@ -710,47 +793,69 @@ __device__ __forceinline__ SplitFactors split_factors(float pdf, float w, float 
   return {ip, cf, wip};
 }
 
-// The staged chunk's samples s = quad, quad + 64, ... in that order, for the
-// first JT component groups with no branch between the components (groups in
-// [J, JT) hold zero-weight components, whose sums are not read).  The frame
-// of component k is one 16 B and one 8 B read of sh.frame[k]; the next
-// group's frame is read while the current group's sums are formed.
+// The staged chunk's samples, four per quad and step, for the first JT
+// component groups with no branch between the components (groups in [J, JT)
+// hold zero-weight components, whose sums are not read).  The coordinates of
+// the four samples in a group's frames are six matrix instructions; the frame
+// of component k is one 16 B and one 8 B read of sh.frame[k], the next group's
+// read while the current group's sums are formed.  A sample the mixture does
+// not cover adds zero.
 template <int JT>
-__device__ __forceinline__ void split_chunk(const Shared& sh, const CompRegs& c, int q, int quad, uint32_t cnt,
-                                            float inv_mc, SplitAcc& a) {
-  for (uint32_t s = quad; s < cnt; s += RT / 4) {
-    const float dx = sh.stage[0][s], dy = sh.stage[1][s], dz = sh.stage[2][s];
-    float e[8];
-    const float pdf = soft_eval_t<JT>(c, dx, dy, dz, e);
-    if (pdf > 1e-16f) {
-      const SplitFactors F = split_factors(pdf, sh.stage[3][s], sh.stage[4][s], inv_mc);
-      a.cnt += 1.f;
-      float4 f0 = *reinterpret_cast<const float4*>(&sh.frame[q][0]);
-      float2 f1 = *reinterpret_cast<const float2*>(&sh.frame[q][4]);
+__device__ __forceinline__ void split_chunk(const Shared& sh, int q, uint32_t cnt, float inv_mc, SplitAcc& a) {
+  const uint32_t tid = threadIdx.x;
+  const uint32_t own = (tid >> 2) + 64u * (uint32_t)q;  // this lane's sample of the first step
+  const Mat4 zero = {0.f, 0.f, 0.f, 0.f};
+  for (uint32_t s0 = 0; s0 < cnt; s0 += RT) {
+    // the component and frame tables are read in every step: 88 registers of
+    // them kept over the loop do not fit beside its 48 sums and spill
+    asm volatile("" ::: "memory");
+    CompRegs c;
 #pragma unroll
-      for (int j = 0; j < JT; j++) {
-        float4 n0 = f0;
-        float2 n1 = f1;
-        if (j + 1 < JT) {
-          n0 = *reinterpret_cast<const float4*>(&sh.frame[4 * (j + 1) + q][0]);
-          n1 = *reinterpret_cast<const float2*>(&sh.frame[4 * (j + 1) + q][4]);
-        }
-        split_add(a, j, f0, f1, dx, dy, dz, e[j], F.ip, F.cf, F.wip);
-        f0 = n0;
-        f1 = n1;
+    for (int j = 0; j < JT; j++) load_comp(sh, q, j, c);
+    const float x = sh.stage[0][s0 + tid], y = sh.stage[1][s0 + tid], z = sh.stage[2][s0 + tid];
+    Mat4 e[8];
+    const float pdf = soft_eval_quad<JT>(c, q, x, y, z, e);
+    const bool ok = pdf > 1e-16f && s0 + own < cnt;
+    SplitFactors F = split_factors(pdf, sh.stage[3][s0 + tid], sh.stage[4][s0 + tid], inv_mc);
+    F.ip = ok ? F.ip : 0.f;
+    F.cf = ok ? F.cf : 0.f;
+    F.wip = ok ? F.wip : 0.f;
+    a.cnt += ok ? 1.f : 0.f;
+    const float ip[4] = {quad_bcast<0>(F.ip), quad_bcast<1>(F.ip), quad_bcast<2>(F.ip), quad_bcast<3>(F.ip)};
+    const float cf[4] = {quad_bcast<0>(F.cf), quad_bcast<1>(F.cf), quad_bcast<2>(F.cf), quad_bcast<3>(F.cf)};
+    const float wip[4] = {quad_bcast<0>(F.wip), quad_bcast<1>(F.wip), quad_bcast<2>(F.wip), quad_bcast<3>(F.wip)};
+    float4 f0 = *reinterpret_cast<const float4*>(&sh.frame[q][0]);
+    float2 f1 = *reinterpret_cast<const float2*>(&sh.frame[q][4]);
+#pragma unroll
+    for (int j = 0; j < JT; j++) {
+      float4 n0 = f0;
+      float2 n1 = f1;
+      if (j + 1 < JT) {
+        n0 = *reinterpret_cast<const float4*>(&sh.frame[4 * (j + 1) + q][0]);
+        n1 = *reinterpret_cast<const float2*>(&sh.frame[4 * (j + 1) + q][4]);
       }
+      Mat4 lx = quad_mfma(z, f0.z, zero), ly = quad_mfma(z, f1.y, zero);
+      lx = quad_mfma(y, f0.y, lx);
+      ly = quad_mfma(y, f1.x, ly);
+      lx = quad_mfma(x, f0.x, lx);
+      ly = quad_mfma(x, f0.w, ly);
+#pragma unroll
+      for (int i = 0; i < 4; i++) split_add(a, j, lx[i], ly[i], e[j][i], ip[i], cf[i], wip[i]);
+      f0 = n0;
+      f1 = n1;
     }
   }
 }
 
 __device__ void pass_split(Shared& sh, Team& tm, const RegionSamples& rs, uint32_t base, uint32_t n, float mcEst) {
   const unsigned long long tPass = wall_clock64();
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = tid & 3, quad = tid >> 2;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, q = tid & 3;
   const VMMParams& V = sh.S.vmm;
   const int K = V.K;
   const int J = (K + 3) >> 2;
-  CompRegs c;
-  load_comps(V, q, c);
+  fill_comps(sh);  // visible to the sample loop behind the barrier after the staging
+  const int vi = sum8_index(lane);
+  const bool odd = (lane & 4) != 0;
   const float inv_mc = 1.f / mcEst;
   float fs = 0.f, fc = 0.f;
   double fd = 0.0;
@@ -766,31 +871,24 @@ __device__ void pass_split(Shared& sh, Team& tm, const RegionSamples& rs, uint32
     for (int j = 0; j < 8; j++) achi[j] = asa[j] = asw[j] = acx[j] = acy[j] = acz[j] = 0.f;
     float cnt = 0.f;
     SplitAcc a{achi, asa, asw, acx, acy, acz, cnt};
-    with_groups(J, [&](auto jt) { split_chunk<decltype(jt)::value>(sh, c, q, quad, ce - cb, inv_mc, a); });
+    with_groups(J, [&](auto jt) {
+      constexpr int JT = decltype(jt)::value;
+      split_chunk<JT>(sh, q, ce - cb, inv_mc, a);
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const float v0 = quad_group_sum(achi[j]);
-      const float v1 = quad_group_sum(asa[j]);
-      const float v2 = quad_group_sum(asw[j]);
-      const float v3 = quad_group_sum(acx[j]);
-      const float v4 = quad_group_sum(acy[j]);
-      const float v5 = quad_group_sum(acz[j]);
-      if (lane < 4) {
-        const int k = 4 * j + lane;
-        sh.red[wave][k][0] = v0;
-        sh.red[wave][k][1] = v1;
-        sh.red[wave][k][2] = v2;
-        sh.red[wave][k][3] = v3;
-        sh.red[wave][k][4] = v4;
-        sh.red[wave][k][5] = v5;
+      for (int j = 0; j < JT; j += 4) {
+#pragma unroll
+        for (int f = 0; f < 6; f += 2) {
+          const float* s0 = f == 0 ? achi : (f == 2 ? asw : acy);
+          const float* s1 = f == 0 ? asa : (f == 2 ? acx : acz);
+          const float s = sum8(odd, s0[j], s1[j], s0[j + 1], s1[j + 1], s0[j + 2], s1[j + 2], s0[j + 3], s1[j + 3]);
+          if ((lane & 8) == 0) sh.red[wave][f + (vi & 1)][4 * (j + (vi >> 1)) + q] = s;
+        }
       }
-    }
-    // every lane of a quad counted the sample: divide the wave sum by 4
-    const float vc = wave_sum0(cnt) * 0.25f;
+    });
+    const float vc = wave_sum0(cnt);  // every lane counted its own samples (whole numbers: exact)
     if (lane == 0) sh.scal[wave][0] = vc;
     __syncthreads();
-    chunk_out(sh, tm, ch, 6, 1, -1, fs, fc, fd);
-    __syncthreads();
+    chunk_out(sh, tm, ch, 6, 1, 4 * J, -1, fs, fc, fd);
   }
   pass_finish(sh, tm, -1, fs, fc, fd);
   if (tid == 0) { sh.S.splitEvals += (float)n * (float)K; sh.S.prof[2] += (float)(wall_clock64() - tPass); }
