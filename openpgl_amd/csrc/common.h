@@ -131,7 +131,7 @@ struct RegionState {
   float splitEvals;     // sample x component evaluations in split-statistics passes
   // profile of the last update (rank 0 of the region's team), wall-clock
   // ticks: [0] total, [1] E-step passes, [2] split passes, [3] distance
-  // passes, [4] team barrier waits, [5] merging, [6] splitting logic,
+  // passes, [4] waits for team partials, [5] merging, [6] splitting logic,
   // [9] M-step and convergence test, [10] cross-chunk folds;
   // counts: [7] team size, [8] E-step passes, [11] samples
   float prof[12];
@@ -162,7 +162,7 @@ struct RegionInput {
 };
 
 // One region of a directional launch: team = workgroups working on it,
-// chunks = ceil(samples / kChunk), partialOffset = float offset of its
+// chunks = ceil(samples / kChunk), partialOffset = 8-byte word offset of its
 // 2 x chunks x kPartStride partial buffer.
 struct RegionJob {
   uint32_t region, team, chunks, pad;

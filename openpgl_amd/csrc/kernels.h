@@ -102,9 +102,9 @@ void launch_knn8(const float4* pivots, uint32_t numRegions, uint32_t* nbIds, flo
 // directional
 // Directional update of the regions listed in jobs (persistent kernel, see
 // kernels_region.hip).  items: (job, rank) pairs, ranks of a job consecutive;
-// queueAndCounters: numJobs + 1 words (cleared by the launcher); partial: per
-// job 2 x chunks x kPartStride floats at job.partialOffset; err: set to 1 when
-// a team barrier waited longer than timeoutTicks of the wall clock
+// queue: one word; partial: per job of a team 2 x chunks x kPartStride 8-byte
+// words at job.partialOffset (both zeroed by launch_prepare_regions); err: set
+// to 1 when a rank waited longer than timeoutTicks of the wall clock
 // (wall_clock64); stats: E-step, distance and split evaluations and EM
 // iterations are added to stats[0..3]; costHint (optional, per region):
 // evaluations per sample of this update.  Every job's team must be <= grid.
@@ -115,8 +115,8 @@ struct RegionLaunch {
   const uint2* items;
   uint32_t numItems;
   uint32_t grid;
-  uint32_t* queueAndCounters;
-  float* partial;
+  uint32_t* queue;
+  unsigned long long* partial;
   int* err;
   unsigned long long timeoutTicks;
   unsigned long long* stats;
@@ -124,7 +124,7 @@ struct RegionLaunch {
   const float *dx, *dy, *dz, *w, *pdf, *dist;
   const float* uniformDirs;
   bool cooperative;
-  bool zeroQueue;  // zero the queue and team counters before the launch (else done by launch_prepare_regions)
+  bool zeroQueue;  // zero the queue before the launch (else done by launch_prepare_regions)
 };
 int region_kernel_blocks_per_cu();
 void launch_region_update(const RegionLaunch& launch, const FactoryConfig& cfg, hipStream_t s);
@@ -133,13 +133,13 @@ void launch_copy_states(RegionState* states, const uint32_t* pairs /* dst, src *
 void launch_set_inputs(RegionState* states, const RegionInput* inputs, uint32_t count, hipStream_t s);
 // One kernel before a persistent region launch, reading its tables from
 // pinned host memory: copies tableBytes (a multiple of 16) from hostTables to
-// tables, zeroes numZero words at zero (queue and team counters), the error
-// flag and the four launch totals; with inputs (host, pinned), every region's
+// tables, zeroes the queue, partialBytes (a multiple of 16) of team partials,
+// the error flag and the four launch totals; with inputs (host, pinned), every region's
 // state is first copied from its ancestor where copyFrom >= 0 and then given
 // its inputs (launch_copy_states followed by launch_set_inputs).
 void launch_prepare_regions(RegionState* states, const void* hostTables, void* tables, size_t tableBytes,
-                            const RegionInput* inputs, uint32_t numInputs, uint32_t* zero, uint32_t numZero, int* err,
-                            unsigned long long* stats, hipStream_t s);
+                            const RegionInput* inputs, uint32_t numInputs, uint32_t* queue, void* partial,
+                            size_t partialBytes, int* err, unsigned long long* stats, hipStream_t s);
 
 // query
 // One piece of a query batch: queries [begin, begin + n) of the batch read

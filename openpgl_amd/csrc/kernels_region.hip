@@ -13,7 +13,8 @@
 // per-region logic on identical LDS state.  Because the chunking and the fold
 // order do not depend on T, the result is bit-identical for every team size
 // and schedule.  Ranks exchange partials through global memory (double
-// buffered) and meet at a counter barrier with a bounded wait.  Work items
+// buffered): every value travels in one 8-byte word with the number of its
+// pass, and the reader waits, boundedly, for the words themselves.  Work items
 // (region, rank) are taken from a queue in order, with every rank of a team
 // queued consecutively, by a grid that is co-resident on the device.
 //
@@ -87,11 +88,10 @@ struct RegionSamples {
 // Team context of a workgroup (kept in LDS; thread 0 advances the epoch).
 struct Team {
   uint32_t rank, T, nc;
-  float* part;          // 2 x nc x kPartStride floats of this region
-  uint32_t* counter;    // barrier counter of this region
-  uint32_t epoch;       // barriers passed
+  unsigned long long* part;  // 2 x nc x kPartStride words of this region
+  uint32_t epoch;       // passes exchanged
   int* err;
-  unsigned long long timeout;  // longest barrier wait, wall-clock ticks
+  unsigned long long timeout;  // longest wait, wall-clock ticks
 };
 
 struct Shared {
@@ -121,7 +121,7 @@ struct Shared {
   int32_t W;  // SIMD width of the emulated reference device
   float fin[kPartStride];  // folded pass results (layout: see the pass functions)
   double finLL;            // folded log-likelihood
-  int32_t abort;           // a team barrier timed out: finish without waiting
+  int32_t abort;           // a wait for team partials timed out: finish without waiting
   uint32_t item;           // queue item of this workgroup
   FactoryConfig cfg;       // launch constants, read from LDS by the region logic
   RegionSamples rs;
@@ -364,54 +364,65 @@ __device__ __forceinline__ void kfold(float& sum, float& comp, float x) {
   sum = t;
 }
 
-// value v of the current chunk from the per-wave partials (fixed order);
-// components from KG on have none (zero)
-__device__ __forceinline__ float chunk_value(const Shared& sh, int v, int F, int NS, int KG) {
-  if (v < 32 * F) {
-    const int f = v >> 5, k = v & 31;
-    if (k >= KG) return 0.f;
-    return (sh.red[0][f][k] + sh.red[1][f][k]) + (sh.red[2][f][k] + sh.red[3][f][k]);
-  }
-  if (v >= kScal && v < kScal + NS) {
-    const int i = v - kScal;
-    return (sh.scal[0][i] + sh.scal[1][i]) + (sh.scal[2][i] + sh.scal[3][i]);
-  }
-  return 0.f;
+// Whether the chunk sums of a pass (F fields of KG components, NS scalars)
+// have a value at place v.
+__device__ __forceinline__ bool value_used(int v, int F, int NS, int KG) {
+  return v < 32 * F ? (v & 31) < KG : (v >= kScal && v < kScal + NS);
 }
 
-// Team barrier.  Partials are written with device-coherent (agent-scope
-// relaxed atomic, write-through) stores and read with device-coherent loads,
-// so no cache writeback or invalidation is needed: each wave waits for its
-// stores to complete (s_waitcnt), the workgroup arrives on the counter and
-// waits until all T ranks have arrived.  The wait is bounded: after
-// tm.timeout ticks of the constant-rate wall clock, or as soon as any
-// workgroup has raised the error flag, the workgroup raises the flag and stops
-// waiting at this and every later barrier (it still arrives, so no teammate
-// waits for it).  The host turns the flag into an error.
-__device__ void team_barrier(Shared& sh, Team& tm) {
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    tm.epoch++;  // read by the other threads after the closing barrier
-    const unsigned long long tb = wall_clock64();
-    atomicAdd(tm.counter, 1u);
-    if (!sh.abort) {
-      const uint32_t target = tm.epoch * tm.T;
-      const unsigned long long t0 = tb;
-      while (__hip_atomic_load(tm.counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
-        __builtin_amdgcn_s_sleep(2);
-        if (__hip_atomic_load(tm.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 ||
-            wall_clock64() - t0 > tm.timeout) {
-          atomicExch(tm.err, 1);
-          sh.abort = 1;
-          break;
-        }
-      }
-    }
-    sh.S.prof[4] += (float)(wall_clock64() - tb);
+// used value v of the current chunk from the per-wave partials (fixed order)
+__device__ __forceinline__ float chunk_value(const Shared& sh, int v, int F) {
+  if (v < 32 * F) {
+    const int f = v >> 5, k = v & 31;
+    return (sh.red[0][f][k] + sh.red[1][f][k]) + (sh.red[2][f][k] + sh.red[3][f][k]);
   }
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-  __syncthreads();
+  const int i = v - kScal;
+  return (sh.scal[0][i] + sh.scal[1][i]) + (sh.scal[2][i] + sh.scal[3][i]);
+}
+
+// Team exchange.  A rank writes every value of its chunks' sums as one 8-byte
+// word, the value and the number of the pass (epoch + 1; the launch starts with
+// zeroed words), with device-coherent (agent-scope relaxed atomic,
+// write-through) stores, and each thread of every rank reads the words of its
+// place until they carry the pass: the wait for a partial is the read of it.
+// (An arrival counter instead costs, on the way of every pass, the wait for the
+// stores, an atomic, the polling of the counter and then the reads: 9 of a
+// pass's 20 us in a team of 12 with two chunks per rank, waits for slower ranks
+// included; a first update of 1 M samples in 48 regions 1.35 -> 1.20 ms.)
+//
+// Two buffers suffice: a rank writes pass e + 2 over pass e only after it has
+// read all ranks' words of pass e + 1, and a rank writes those behind the
+// barrier that ends its reading of pass e.  The wait is bounded: after
+// tm.timeout ticks of the constant-rate wall clock, or as soon as any workgroup
+// has raised the error flag, the workgroup raises the flag and stops waiting in
+// this and every later pass (it still writes its words, so no teammate waits
+// for it).  The host turns the flag into an error.
+__device__ __forceinline__ unsigned long long part_load(const unsigned long long* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Waits until *p carries the pass `tag` in every active lane; false once the
+// workgroup no longer waits.
+__device__ __forceinline__ bool part_wait(Shared& sh, const Team& tm, const unsigned long long* p, uint32_t tag) {
+  const unsigned long long t0 = wall_clock64();
+  bool ok = true;
+  for (;;) {
+    if (__ballot((uint32_t)(part_load(p) >> 32) != tag) == 0) break;
+    if (__hip_atomic_load(&sh.abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != 0) {
+      ok = false;
+      break;
+    }
+    if (__hip_atomic_load(tm.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 ||
+        wall_clock64() - t0 > tm.timeout) {
+      atomicExch(tm.err, 1);
+      __hip_atomic_store(&sh.abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      ok = false;
+      break;
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+  if (threadIdx.x == 0) sh.S.prof[4] += (float)(wall_clock64() - t0);
+  return ok;
 }
 
 // End of a chunk: value v = threadIdx.x of chunk c goes into the running fold
@@ -421,45 +432,81 @@ __device__ void team_barrier(Shared& sh, Team& tm) {
 __device__ __forceinline__ void chunk_out(const Shared& sh, const Team& tm, uint32_t c, int F, int NS, int KG,
                                           int llIdx, float& fs, float& fc, double& fd) {
   const int v = threadIdx.x;
-  const float x = chunk_value(sh, v, F, NS, KG);
+  if (!value_used(v, F, NS, KG)) return;
+  const float x = chunk_value(sh, v, F);
   if (tm.T == 1) {
     if (v == llIdx) fd += (double)x;
     else kfold(fs, fc, x);
   } else {
-    __hip_atomic_store(tm.part + ((size_t)(tm.epoch & 1u) * tm.nc + c) * kPartStride + v, x, __ATOMIC_RELAXED,
+    const uint32_t tag = tm.epoch + 1u;
+    const unsigned long long w = ((unsigned long long)tag << 32) | __float_as_uint(x);
+    __hip_atomic_store(tm.part + ((size_t)(tm.epoch & 1u) * tm.nc + c) * kPartStride + v, w, __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
-// End of a pass: fold the chunk partials of all ranks in chunk order, publish in sh.fin.
-__device__ void pass_finish(Shared& sh, Team& tm, int llIdx, float fs, float fc, double fd) {
+// The chunk partials of all ranks at this thread's place, folded in chunk
+// order (out of line: its registers are not the sample passes').
+struct Folded {
+  float f;
+  double d;
+};
+__device__ __noinline__ Folded team_fold(Shared& sh, const Team& tm, int F, int NS, int KG, int llIdx) {
   const int v = threadIdx.x;
-  if (tm.T > 1) {
-    const uint32_t buf = tm.epoch & 1u;
-    team_barrier(sh, tm);
+  float fs = 0.f, fc = 0.f;
+  double fd = 0.0;
+  if (value_used(v, F, NS, KG)) {
     const unsigned long long tF = wall_clock64();
-    const float* p = tm.part + (size_t)buf * tm.nc * kPartStride + v;
-    // eight loads in flight at a time, folded in chunk order
-    for (uint32_t c0 = 0; c0 < tm.nc; c0 += 8) {
-      float x[8];
+    const float waited = v == 0 ? sh.S.prof[4] : 0.f;
+    const uint32_t tag = tm.epoch + 1u, nc = tm.nc;
+    const unsigned long long* p = tm.part + (size_t)(tm.epoch & 1u) * nc * kPartStride + v;
+    bool wait = true;
+    // kFold loads in flight at a time
+    constexpr uint32_t kFold = 16;
+    for (uint32_t c0 = 0; c0 < nc; c0 += kFold) {
+      unsigned long long w[kFold];
 #pragma unroll
-      for (int u = 0; u < 8; u++)
-        x[u] = c0 + u < tm.nc ? __hip_atomic_load(p + (size_t)(c0 + u) * kPartStride, __ATOMIC_RELAXED,
-                                                  __HIP_MEMORY_SCOPE_AGENT)
-                              : 0.f;
+      for (uint32_t u = 0; u < kFold; u++) w[u] = c0 + u < nc ? part_load(p + (size_t)(c0 + u) * kPartStride) : 0ull;
+      while (wait) {
+        // the words that have not arrived (uniform over the wave): wait for the first, then read them again
+        uint32_t late = 0;
 #pragma unroll
-      for (int u = 0; u < 8; u++) {
-        if (c0 + u < tm.nc) {
-          if (v == llIdx) fd += (double)x[u];
-          else kfold(fs, fc, x[u]);
+        for (uint32_t u = 0; u < kFold; u++)
+          late |= (c0 + u < nc && __ballot((uint32_t)(w[u] >> 32) != tag) != 0) ? 1u << u : 0u;
+        if (late == 0) break;
+        wait = part_wait(sh, tm, p + (size_t)(c0 + __builtin_ctz(late)) * kPartStride, tag);
+#pragma unroll
+        for (uint32_t u = 0; u < kFold; u++)
+          if ((late >> u) & 1u) w[u] = part_load(p + (size_t)(c0 + u) * kPartStride);
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < kFold; u++) {
+        if (c0 + u < nc) {
+          const float x = __uint_as_float((uint32_t)w[u]);
+          if (v == llIdx) fd += (double)x;
+          else kfold(fs, fc, x);
         }
       }
     }
-    if (v == 0) sh.S.prof[10] += (float)(wall_clock64() - tF);
+    if (v == 0) sh.S.prof[10] += (float)(wall_clock64() - tF) - (sh.S.prof[4] - waited);
+  }
+  return {fs, fd};
+}
+
+// End of a pass: the folded sums (of a team: of all ranks' chunks) into sh.fin.
+__device__ __forceinline__ void pass_finish(Shared& sh, Team& tm, int F, int NS, int KG, int llIdx, float fs,
+                                            double fd) {
+  const int v = threadIdx.x;
+  const bool team = tm.T > 1;
+  if (team) {
+    const Folded r = team_fold(sh, tm, F, NS, KG, llIdx);
+    fs = r.f;
+    fd = r.d;
   }
   sh.fin[v] = fs;
   if (v == llIdx) sh.finLL = fd;
   __syncthreads();
+  if (team && v == 0) tm.epoch++;  // read again behind a later barrier
 }
 
 // Place of sample o of a chunk in the staging arrays: quad p of the workgroup
@@ -670,7 +717,7 @@ __device__ __forceinline__ void pass_estep(Shared& sh, Team& tm, const RegionSam
     __syncthreads();
     chunk_out(sh, tm, ch, 4, 5, 4 * J, kScal, fs, fc, fd);
   }
-  pass_finish(sh, tm, kScal, fs, fc, fd);
+  pass_finish(sh, tm, 4, 5, 4 * J, kScal, fs, fd);
   if (tid == 0) {
     sh.S.estepEvals += (float)n * (float)K;
     sh.S.prof[1] += (float)(wall_clock64() - tPass);
@@ -750,7 +797,7 @@ __device__ void pass_distances(Shared& sh, Team& tm, const RegionSamples& rs, ui
     __syncthreads();
     chunk_out(sh, tm, ch, 2, 0, 4 * J, -1, fs, fc, fd);
   }
-  pass_finish(sh, tm, -1, fs, fc, fd);
+  pass_finish(sh, tm, 2, 0, 4 * J, -1, fs, fd);
   if (tid == 0) { sh.S.auxEvals += (float)n * (float)K; sh.S.prof[3] += (float)(wall_clock64() - tPass); }
 }
 
@@ -894,7 +941,7 @@ __device__ void pass_split(Shared& sh, Team& tm, const RegionSamples& rs, uint32
     __syncthreads();
     chunk_out(sh, tm, ch, 6, 1, 4 * J, -1, fs, fc, fd);
   }
-  pass_finish(sh, tm, -1, fs, fc, fd);
+  pass_finish(sh, tm, 6, 1, 4 * J, -1, fs, fd);
   if (tid == 0) { sh.S.splitEvals += (float)n * (float)K; sh.S.prof[2] += (float)(wall_clock64() - tPass); }
 }
 
@@ -1954,8 +2001,8 @@ __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(PGL_REG
 PGL_REGION_KERNEL(RegionState* __restrict__ states,
                                                       const RegionJob* __restrict__ jobs,
                                                       const uint2* __restrict__ items, uint32_t numItems,
-                                                      uint32_t* __restrict__ queue, uint32_t* __restrict__ counters,
-                                                      float* __restrict__ partial, int* __restrict__ err,
+                                                      uint32_t* __restrict__ queue,
+                                                      unsigned long long* __restrict__ partial, int* __restrict__ err,
                                                       unsigned long long timeout,
                                                       unsigned long long* __restrict__ stats,
                                                       float* __restrict__ costHint, RegionSamples rs,
@@ -1982,7 +2029,6 @@ PGL_REGION_KERNEL(RegionState* __restrict__ states,
         tm.T = job.team;
         tm.nc = job.chunks;
         tm.part = partial + job.partialOffset;
-        tm.counter = counters + item.x;
         tm.epoch = 0;
         tm.err = err;
         tm.timeout = timeout;
@@ -2043,20 +2089,23 @@ __global__ void __launch_bounds__(256) k_set_inputs(RegionState* __restrict__ st
 
 // Reads the launch's tables straight from pinned host memory (no copy
 // operation before it): all blocks copy the job and item tables (copy16
-// 16-byte words) to device memory for the region kernel; block 0 zeroes the
-// launch's counters; block b < numInputs prepares the region of inputs[b].  A
+// 16-byte words) to device memory for the region kernel and zero the teams'
+// partial words; block 0 zeroes the launch's counters; block b < numInputs prepares the region of inputs[b].  A
 // new region's ancestor may receive its own inputs while the copy runs: only
 // input fields can differ, and the new region overwrites all of them.
 __global__ void __launch_bounds__(256) k_prepare_regions(RegionState* __restrict__ states,
                                                          const uint4* __restrict__ hostTables, uint4* __restrict__ tables,
                                                          uint32_t copy16, const RegionInput* __restrict__ in,
-                                                         uint32_t numInputs, uint32_t* __restrict__ zero,
-                                                         uint32_t numZero, int* __restrict__ err,
+                                                         uint32_t numInputs, uint32_t* __restrict__ queue,
+                                                         uint4* __restrict__ partial, uint32_t partial16,
+                                                         int* __restrict__ err,
                                                          unsigned long long* __restrict__ stats) {
   const uint32_t b = blockIdx.x;
+  for (uint32_t i = b * blockDim.x + threadIdx.x; i < partial16; i += gridDim.x * blockDim.x)
+    partial[i] = make_uint4(0u, 0u, 0u, 0u);
   for (uint32_t i = b * blockDim.x + threadIdx.x; i < copy16; i += gridDim.x * blockDim.x) tables[i] = hostTables[i];
   if (b == 0) {
-    for (uint32_t i = threadIdx.x; i < numZero; i += blockDim.x) zero[i] = 0u;
+    if (threadIdx.x == 0 && queue) *queue = 0u;
     if (threadIdx.x == 0) *err = 0;
     if (threadIdx.x < 4) stats[threadIdx.x] = 0ull;
   }
@@ -2083,13 +2132,14 @@ __global__ void __launch_bounds__(256) k_prepare_regions(RegionState* __restrict
 }
 
 void launch_prepare_regions(RegionState* states, const void* hostTables, void* tables, size_t tableBytes,
-                            const RegionInput* inputs, uint32_t numInputs, uint32_t* zero, uint32_t numZero, int* err,
-                            unsigned long long* stats, hipStream_t s) {
-  const uint32_t copy16 = (uint32_t)((tableBytes + 15) / 16);
+                            const RegionInput* inputs, uint32_t numInputs, uint32_t* queue, void* partial,
+                            size_t partialBytes, int* err, unsigned long long* stats, hipStream_t s) {
+  const uint32_t copy16 = (uint32_t)((tableBytes + 15) / 16), partial16 = (uint32_t)(partialBytes / 16);
   uint32_t blocks = inputs && numInputs ? numInputs : 1u;
   blocks = std::max<uint32_t>(blocks, std::min<uint32_t>((copy16 + 255) / 256, 1024u));
+  blocks = std::max<uint32_t>(blocks, std::min<uint32_t>((partial16 + 1023) / 1024, 2048u));
   hipLaunchKernelGGL(k_prepare_regions, dim3(blocks), dim3(256), 0, s, states, (const uint4*)hostTables,
-                     (uint4*)tables, copy16, inputs, numInputs, zero, numZero, err, stats);
+                     (uint4*)tables, copy16, inputs, numInputs, queue, (uint4*)partial, partial16, err, stats);
 }
 
 void launch_copy_states(RegionState* states, const uint32_t* pairs, uint32_t numPairs, hipStream_t s) {
@@ -2115,16 +2165,14 @@ int region_kernel_blocks_per_cu() {
 
 void launch_region_update(const RegionLaunch& L, const FactoryConfig& cfg, hipStream_t s) {
   if (L.numItems == 0) return;
-  const uint32_t nz = L.numJobs + 1;
-  if (L.zeroQueue) hipLaunchKernelGGL(k_zero_u32, dim3((nz + 255) / 256), dim3(256), 0, s, L.queueAndCounters, nz);
+  if (L.zeroQueue) hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, L.queue, 1u);
   RegionSamples rs{L.dx, L.dy, L.dz, L.w, L.pdf, L.dist};
   RegionState* states = L.states;
   const RegionJob* jobs = L.jobs;
   const uint2* items = L.items;
   uint32_t numItems = L.numItems;
-  uint32_t* queue = L.queueAndCounters;
-  uint32_t* counters = L.queueAndCounters + 1;
-  float* partial = L.partial;
+  uint32_t* queue = L.queue;
+  unsigned long long* partial = L.partial;
   int* err = L.err;
   unsigned long long timeout = L.timeoutTicks;
   unsigned long long* stats = L.stats;
@@ -2136,8 +2184,8 @@ void launch_region_update(const RegionLaunch& L, const FactoryConfig& cfg, hipSt
   PGL_KERNEL_CHECK(hipGetDevice(&dev));
   PGL_KERNEL_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
   const bool wide = L.grid <= (uint32_t)cus;
-  void* args[] = {&states, &jobs,    &items, &numItems, &queue, &counters,   &partial,
-                  &err,    &timeout, &stats, &costHint, &rs,    (void*)&c, &uniformDirs};
+  void* args[] = {&states, &jobs,  &items,    &numItems, &queue,    &partial,    &err,
+                  &timeout, &stats, &costHint, &rs,       (void*)&c, &uniformDirs};
   const void* fn = wide ? region_kernel_wide() : (const void*)k_region_update;
   if (L.cooperative) PGL_KERNEL_CHECK(hipLaunchCooperativeKernel(fn, dim3(L.grid), dim3(RT), args, 0, s));
   else PGL_KERNEL_CHECK(hipLaunchKernel(fn, dim3(L.grid), dim3(RT), args, 0, s));

@@ -123,7 +123,7 @@ void RegionRunner::stage(std::vector<RegionWork> work, const RegionSamplesView& 
 
   jobs_.resize(J);
   items_.clear();
-  unsigned long long partialFloats = 0;
+  unsigned long long partialWords = 0;
   for (uint32_t j = 0; j < J; j++) {
     const uint32_t n = work[j].samples;
     RegionJob& jb = jobs_[j];
@@ -140,8 +140,8 @@ void RegionRunner::stage(std::vector<RegionWork> work, const RegionSamplesView& 
     }
     jb.team = T;
     jb.pad = 0;
-    jb.partialOffset = T > 1 ? partialFloats : 0ull;
-    if (T > 1) partialFloats += 2ull * jb.chunks * kPartStride;
+    jb.partialOffset = T > 1 ? partialWords : 0ull;
+    if (T > 1) partialWords += 2ull * jb.chunks * kPartStride;
     stagedMaxTeam_ = std::max(stagedMaxTeam_, T);
     if (!perRegion || perRegionTeams)
       for (uint32_t r = 0; r < T; r++) items_.push_back(make_uint2(j, r));
@@ -156,12 +156,12 @@ void RegionRunner::stage(std::vector<RegionWork> work, const RegionSamplesView& 
   // a buffer that grows is freed: first wait until the last launch (and with
   // it every earlier one on its stream), which may still be queued or
   // running and reading it, has completed
-  const size_t partB = std::max<unsigned long long>(partialFloats, 1) * 4;
-  if (submitted_ && (offIn > stageBytes_ || size_t(J + 1) * 4 > queueBytes_ || partB > partialBytes_ ||
+  const size_t partB = std::max<unsigned long long>(partialWords, 1) * sizeof(unsigned long long);
+  if (submitted_ && (offIn > stageBytes_ || sizeof(uint32_t) > queueBytes_ || partB > partialBytes_ ||
                      stageB > hStageBytes_))
     PGL_SCHED_CHECK(hipEventSynchronize(evEnd_[cur_]));
   grow(dStage_, stageBytes_, offIn);
-  grow(dQueue_, queueBytes_, (size_t)(J + 1) * 4);
+  grow(dQueue_, queueBytes_, sizeof(uint32_t));
   grow(dPartial_, partialBytes_, partB);
   grow_pinned(hStage_, hStageBytes_, stageB);
   char* hs = (char*)hStage_;
@@ -173,6 +173,7 @@ void RegionRunner::stage(std::vector<RegionWork> work, const RegionSamplesView& 
   st.offItems = offItems;
   st.offIn = offIn;
   st.inB = inB;
+  st.partialBytes = partialWords * sizeof(unsigned long long);
   st.perRegion = perRegion;
   st.perRegionTeams = perRegionTeams;
 }
@@ -196,8 +197,8 @@ void RegionRunner::submit(RegionState* states, hipStream_t s) {
   char* hdev = (char*)hStageDev_;
   if (st.empty) {
     if (st.numInputs) {
-      launch_prepare_regions(states, nullptr, nullptr, 0, (const RegionInput*)hdev, st.numInputs, nullptr, 0, dErr_,
-                             (unsigned long long*)dStats_, s);
+      launch_prepare_regions(states, nullptr, nullptr, 0, (const RegionInput*)hdev, st.numInputs, nullptr, nullptr, 0,
+                             dErr_, (unsigned long long*)dStats_, s);
       PGL_SCHED_CHECK(hipEventRecord(evPrep_, s));
       prepQueued_ = true;
     }
@@ -209,7 +210,8 @@ void RegionRunner::submit(RegionState* states, hipStream_t s) {
   const uint32_t J = st.J;
   char* ds = (char*)dStage_;
   launch_prepare_regions(states, hdev, ds, st.offIn, st.inB ? (const RegionInput*)(hdev + st.offIn) : nullptr,
-                         st.inB ? st.numInputs : 0, (uint32_t*)dQueue_, J + 1, dErr_, (unsigned long long*)dStats_, s);
+                         st.inB ? st.numInputs : 0, (uint32_t*)dQueue_, dPartial_, st.partialBytes, dErr_,
+                         (unsigned long long*)dStats_, s);
   PGL_SCHED_CHECK(hipEventRecord(evPrep_, s));
   prepQueued_ = true;
 
@@ -221,8 +223,8 @@ void RegionRunner::submit(RegionState* states, hipStream_t s) {
   L.items = (const uint2*)(ds + st.offItems);
   L.numItems = (uint32_t)items_.size();
   L.grid = std::min<uint32_t>(st.G, L.numItems);
-  L.queueAndCounters = (uint32_t*)dQueue_;
-  L.partial = (float*)dPartial_;
+  L.queue = (uint32_t*)dQueue_;
+  L.partial = (unsigned long long*)dPartial_;
   L.err = dErr_;
   L.timeoutTicks = timeoutTicks_;
   L.stats = (unsigned long long*)dStats_;
@@ -233,7 +235,7 @@ void RegionRunner::submit(RegionState* states, hipStream_t s) {
   L.zeroQueue = st.perRegion;
   PGL_SCHED_CHECK(hipEventRecord(evBegin_[k], s));
   if (st.perRegionTeams) {
-    // one launch per job: its consecutive items, the queue and counters zeroed before each
+    // one launch per job: its consecutive items, the queue zeroed before each
     L.cooperative = false;
     L.zeroQueue = true;
     const uint2* allItems = L.items;
@@ -286,7 +288,7 @@ void RegionRunner::check(int slot) const {
     throw std::runtime_error("directional update: failure injected for testing");
   }
   if (hTot_[slot].err != 0)
-    throw std::runtime_error("directional update: a region team barrier timed out (workgroups not co-resident)");
+    throw std::runtime_error("directional update: a wait for team partials timed out (workgroups not co-resident)");
 }
 
 }  // namespace pglgpu

@@ -75,7 +75,7 @@ class RegionRunner {
              uint32_t numInputs = 0);
   void submit(RegionState* states, hipStream_t s);
   int lastSlot() const { return cur_; }
-  // after the launch has completed: throws if a team barrier timed out
+  // after the launch has completed: throws if a wait for team partials timed out
   void check(int slot) const;
   void check() const { check(cur_); }
   // testing: the next check() reports a failed launch (the kernels run normally)
@@ -128,7 +128,7 @@ class RegionRunner {
     const float* uniformDirs = nullptr;
     float* costHint = nullptr;
     uint32_t numInputs = 0, J = 0, G = 0;
-    size_t offItems = 0, offIn = 0, inB = 0;
+    size_t offItems = 0, offIn = 0, inB = 0, partialBytes = 0;
     bool perRegion = false, perRegionTeams = false;
   } staged_;
   uint32_t stagedMaxTeam_ = 0;
