@@ -111,6 +111,8 @@ struct Shared {
                                        // at stage_pos() of the sample's place in the chunk
   uint32_t stageKey;       // first sample (absolute index) of the chunk held in stage[0..3], ~0: none
   uint32_t stageCnt;       // its samples
+  uint32_t stageOdd;       // first sample of the last staged chunk with a direction out of range (~0: none)
+  int32_t compOdd;         // a component parameter is out of range
   const float* stageExtra; // the array whose values stage[4] holds for that chunk (null: none)
   double prevLL, invPrevLL;
   uint32_t mask;
@@ -200,6 +202,11 @@ __device__ __forceinline__ void split_zero_slot(SplitStatsState& s, int k) {
 __device__ __forceinline__ int vec_lim(int W, int K) { int l = ((K + W - 1) / W) * W; return l > 32 ? 32 : l; }
 
 // ------------------------------------------------------------ sample passes
+// Directions and component parameters below this in magnitude give finite
+// exponents (kParamMax^3 is finite); others, NaN included, take the loops that
+// bound the exponent itself (soft_eval_quad).
+static const float kParamMax = 1e12f;
+
 // Component parameters of a pass, as the sample loops read them: one row per
 // component (zero weight from K on).  Callers synchronise before reading.
 __device__ __forceinline__ void fill_comps(Shared& sh, int K) {
@@ -213,6 +220,9 @@ __device__ __forceinline__ void fill_comps(Shared& sh, int K) {
     c[2] = a ? V.muz[k] : 1.f;
     c[3] = a ? V.kappa[k] * 1.44269504088896341f : 0.f;  // kappa log2(e)
     c[4] = a ? V.w[k] * V.norm[k] : 0.f;
+    const bool ok = fabsf(c[0]) + fabsf(c[1]) + fabsf(c[2]) < kParamMax && fabsf(c[3]) < kParamMax;
+    const bool odd = __ballot(!ok) != 0;
+    if (k == 0) sh.compOdd = odd ? 1 : 0;
   }
 }
 
@@ -230,16 +240,23 @@ __device__ __forceinline__ void load_comp(const Shared& sh, int q, int j, CompRe
   c.wn[j] = sh.comp[4 * j + q][4];
 }
 
-// Calls f with std::integral_constant<int, JT> for the smallest even JT >= J
-// (J = component groups in use), so that the sample loops are unrolled over
-// a fixed number of groups with no branch between components; the groups in
-// [J, JT) hold zero-weight components.
+// Calls f(JT, Bounded) for the component groups in use (J), so that the sample
+// loops are unrolled over a fixed number of groups with no branch between
+// components.  With a parameter out of range the loop is the one of eight
+// groups whose exponents are bounded (groups from J on hold zero-weight
+// components).
 template <class F>
-__device__ __forceinline__ void with_groups(int J, F&& f) {
-  if (J > 6) f(std::integral_constant<int, 8>());
-  else if (J > 4) f(std::integral_constant<int, 6>());
-  else if (J > 2) f(std::integral_constant<int, 4>());
-  else f(std::integral_constant<int, 2>());
+__device__ __forceinline__ void with_groups(int J, bool bounded, F&& f) {
+  if (bounded) return f(std::integral_constant<int, 8>(), std::true_type());
+  switch (J) {
+    case 8: return f(std::integral_constant<int, 8>(), std::false_type());
+    case 7: return f(std::integral_constant<int, 7>(), std::false_type());
+    case 6: return f(std::integral_constant<int, 6>(), std::false_type());
+    case 5: return f(std::integral_constant<int, 5>(), std::false_type());
+    case 4: return f(std::integral_constant<int, 4>(), std::false_type());
+    case 3: return f(std::integral_constant<int, 3>(), std::false_type());
+    default: return f(std::integral_constant<int, 2>(), std::false_type());
+  }
 }
 
 // Matrix-core form of a quad's work.  v_mfma_f32_4x4x1_16b_f32 works on 16
@@ -283,8 +300,10 @@ __device__ __forceinline__ float quad_sum_own(int q, const float v[4]) {
 // component k = 4j + q for the quad's sample i (the sample whose direction is
 // x, y, z in lane i), evaluated as w_k norm_k 2^min(kap2_k mu_k.d - kap2_k, 0),
 // with no branch between the components; returns the pdf of the lane's own
-// sample.
-template <int JT>
+// sample.  For a finite exponent x the clamp of 2^x to [0, 1], which the
+// exponential instruction takes along, is 2^min(x, 0) (compared for every
+// float); BOUND takes the minimum itself, for which a NaN exponent counts as 0.
+template <int JT, bool BOUND>
 __device__ __forceinline__ float soft_eval_quad(const CompRegs& c, int q, float x, float y, float z, Mat4 e[8]) {
   float part[4] = {0.f, 0.f, 0.f, 0.f};
   const Mat4 zero = {0.f, 0.f, 0.f, 0.f};
@@ -298,7 +317,10 @@ __device__ __forceinline__ float soft_eval_quad(const CompRegs& c, int q, float 
   for (int j = 0; j < JT; j++) {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      e[j][i] = c.wn[j] * __builtin_amdgcn_exp2f(fminf(fmaf(c.kap2[j], e[j][i], -c.kap2[j]), 0.f));
+      const float ex = fmaf(c.kap2[j], e[j][i], -c.kap2[j]);
+      const float v = BOUND ? __builtin_amdgcn_exp2f(fminf(ex, 0.f))
+                            : __builtin_amdgcn_fmed3f(__builtin_amdgcn_exp2f(ex), 0.f, 1.f);
+      e[j][i] = c.wn[j] * v;
       part[i] += e[j][i];
     }
   }
@@ -559,6 +581,7 @@ __device__ __forceinline__ void stage_chunk(Shared& sh, const RegionSamples& rs,
     if (o < padded) {
       const uint32_t p = stage_pos(o);
       if (loadMain) {
+        if (!(fabsf(v[m][0]) + fabsf(v[m][1]) + fabsf(v[m][2]) < kParamMax)) sh.stageOdd = first;
 #pragma unroll
         for (int a = 0; a < 4; a++) sh.stage[a][p] = v[m][a];
       }
@@ -621,7 +644,7 @@ __device__ __forceinline__ void estep_unassigned(EStepAcc& a, float x, float y, 
 // sums.
 //
 // Bound by the vector unit: per step a lane evaluates 4 JT exponentials, each
-// with a fused multiply-add, a minimum, a product and an addition beside it;
+// with a fused multiply-add, a product and an addition beside it;
 // what is per sample (logarithm, reciprocal) is done by one lane per sample,
 // and the 7 JT multiply-accumulate groups are matrix instructions: 319
 // instructions per 64 samples and 32 components, 1110 with the dot products
@@ -629,7 +652,7 @@ __device__ __forceinline__ void estep_unassigned(EStepAcc& a, float x, float y, 
 // With the chunk sums below, a first update of 8 M samples (363 regions) takes
 // 6.3 instead of 9.4 ms in the region kernel, the next one 2.4 instead of 3.2,
 // bit for bit the same.
-template <int JT>
+template <int JT, bool BOUND>
 __device__ __forceinline__ void estep_chunk(const Shared& sh, const CompRegs& c, int q, uint32_t cnt, EStepAcc& a) {
   const uint32_t tid = threadIdx.x;
   for (uint32_t s0 = 0; s0 < cnt; s0 += RT) {
@@ -640,7 +663,7 @@ __device__ __forceinline__ void estep_chunk(const Shared& sh, const CompRegs& c,
     const bool one = q == 3;
     const float g0 = one ? 1.f : row.x, g1 = one ? 1.f : row.y, g2 = one ? 1.f : row.z, g3 = one ? 1.f : row.w;
     Mat4 e[8];
-    const float pdf = soft_eval_quad<JT>(c, q, x, y, z, e);
+    const float pdf = soft_eval_quad<JT, BOUND>(c, q, x, y, z, e);
     const bool ok = pdf > 1e-16f;
     const float lw = ok ? w : 0.f, lp = ok ? logf(pdf) : 0.f;
     const float r = ok ? w * __builtin_amdgcn_rcpf(pdf) : 0.f;
@@ -701,9 +724,10 @@ __device__ __forceinline__ void pass_estep(Shared& sh, Team& tm, const RegionSam
 #pragma unroll
     for (int j = 0; j < 8; j++) a.b[j] = Mat4{0.f, 0.f, 0.f, 0.f};
     a.ll = a.u0 = a.u1 = a.u2 = a.u3 = 0.f;
-    with_groups(J, [&](auto jt) {
+    with_groups(J, sh.compOdd != 0 || sh.stageOdd == base + cb, [&](auto jt, auto bt) {
       constexpr int JT = decltype(jt)::value;
-      estep_chunk<JT>(sh, c, q, ce - cb, a);
+      constexpr bool BOUND = decltype(bt)::value;
+      estep_chunk<JT, BOUND>(sh, c, q, ce - cb, a);
 #pragma unroll
       for (int j = 0; j < JT; j += 2) {
         const Mat4 b0 = a.b[j], b1 = a.b[j + 1];
@@ -759,13 +783,14 @@ __device__ void pass_distances(Shared& sh, Team& tm, const RegionSamples& rs, ui
 #pragma unroll
     for (int j = 0; j < 8; j++) acc[j] = Mat4{0.f, 0.f, 0.f, 0.f};
     const uint32_t cnt = ce - cb;
-    with_groups(J, [&](auto jt) {
+    with_groups(J, sh.compOdd != 0 || sh.stageOdd == base + cb, [&](auto jt, auto bt) {
       constexpr int JT = decltype(jt)::value;
+      constexpr bool BOUND = decltype(bt)::value;
       for (uint32_t s0 = 0; s0 < cnt; s0 += RT) {
         const float x = sh.stage[0][s0 + tid], y = sh.stage[1][s0 + tid], z = sh.stage[2][s0 + tid];
         const float w = sh.stage[3][s0 + tid];
         Mat4 e[8];
-        const float pdf = soft_eval_quad<JT>(c, q, x, y, z, e);
+        const float pdf = soft_eval_quad<JT, BOUND>(c, q, x, y, z, e);
         const bool ok = pdf > 1e-16f;  // other samples add zero
         // w g_k (g_k pdf / w_k) = (w / pdf) e_k^2 / w_k; 1 / w_k is applied to the chunk sums
         const float dist = sh.stage[4][s0 + tid];
@@ -851,7 +876,7 @@ __device__ __forceinline__ SplitFactors split_factors(float pdf, float w, float 
 // of component k is one 16 B and one 8 B read of sh.frame[k], the next group's
 // read while the current group's sums are formed.  A sample the mixture does
 // not cover adds zero.
-template <int JT>
+template <int JT, bool BOUND>
 __device__ __forceinline__ void split_chunk(const Shared& sh, int q, uint32_t cnt, float inv_mc, SplitAcc& a) {
   const uint32_t tid = threadIdx.x;
   const uint32_t own = (tid >> 2) + 64u * (uint32_t)q;  // this lane's sample of the first step
@@ -865,7 +890,7 @@ __device__ __forceinline__ void split_chunk(const Shared& sh, int q, uint32_t cn
     for (int j = 0; j < JT; j++) load_comp(sh, q, j, c);
     const float x = sh.stage[0][s0 + tid], y = sh.stage[1][s0 + tid], z = sh.stage[2][s0 + tid];
     Mat4 e[8];
-    const float pdf = soft_eval_quad<JT>(c, q, x, y, z, e);
+    const float pdf = soft_eval_quad<JT, BOUND>(c, q, x, y, z, e);
     const bool ok = pdf > 1e-16f && s0 + own < cnt;
     SplitFactors F = split_factors(pdf, sh.stage[3][s0 + tid], sh.stage[4][s0 + tid], inv_mc);
     F.ip = ok ? F.ip : 0.f;
@@ -922,9 +947,10 @@ __device__ void pass_split(Shared& sh, Team& tm, const RegionSamples& rs, uint32
     for (int j = 0; j < 8; j++) achi[j] = asa[j] = asw[j] = acx[j] = acy[j] = acz[j] = 0.f;
     float cnt = 0.f;
     SplitAcc a{achi, asa, asw, acx, acy, acz, cnt};
-    with_groups(J, [&](auto jt) {
+    with_groups(J, sh.compOdd != 0 || sh.stageOdd == base + cb, [&](auto jt, auto bt) {
       constexpr int JT = decltype(jt)::value;
-      split_chunk<JT>(sh, q, ce - cb, inv_mc, a);
+      constexpr bool BOUND = decltype(bt)::value;
+      split_chunk<JT, BOUND>(sh, q, ce - cb, inv_mc, a);
 #pragma unroll
       for (int j = 0; j < JT; j += 4) {
 #pragma unroll
@@ -2015,6 +2041,7 @@ PGL_REGION_KERNEL(RegionState* __restrict__ states,
     sh.rs = rs;
     sh.stageKey = 0xffffffffu;
     sh.stageCnt = 0;
+    sh.stageOdd = 0xffffffffu;
     sh.stageExtra = nullptr;
   }
   for (;;) {
