@@ -365,10 +365,13 @@ size_t pglFieldGetUpdateHistory(PGLField field, int kind, double* out, size_t ma
  *                      maxTeam and the device), each region alone on the
  *                      device; 0: one persistent launch
  *   grid               workgroups of the persistent launch (0: two per CU,
- *                      which leaves room for other streams' kernels; at
- *                      most the workgroups that fit at once, three per CU)
+ *                      which leaves room for other streams' kernels, and
+ *                      most of the three that fit for launches of more
+ *                      regions or 1024-sample chunks than those can share;
+ *                      at most the workgroups that fit at once)
  *   balance            a team gets one workgroup per
- *                      total samples / (grid * balance) of its region
+ *                      total samples / (grid * balance) of its region (with
+ *                      grid 0 and many chunks per workgroup, half of that)
  *   minChunksPerRank   at least this many 1024-sample chunks per workgroup
  *   maxTeam            largest team
  *   cooperative        1: cooperative launch (the runtime guarantees that the

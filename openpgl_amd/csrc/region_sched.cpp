@@ -16,6 +16,13 @@ namespace pglgpu {
                                                    " in " #expr);                                         \
   } while (0)
 
+// chunks per workgroup of the default grid from which a launch is bound by throughput
+static const uint64_t kManyChunks = 6;
+// workgroups that a launch bound by throughput leaves to another field's launch
+// beside it: the largest team of the default schedule, so that such a team is
+// always resident as a whole and none waits for the end of this launch
+static const uint32_t kLeaveGroups = 64;
+
 static void grow_pinned(void*& p, size_t& have, size_t need) {
   if (need <= have) return;
   if (p) PGL_SCHED_CHECK(hipHostFree(p));
@@ -113,10 +120,29 @@ void RegionRunner::stage(std::vector<RegionWork> work, const RegionSamplesView& 
   // and the resident grid), i.e. each region alone on the device
   const bool perRegion = schedule.perRegionLaunches != 0;
   const bool perRegionTeams = schedule.perRegionLaunches == 2;
-  const uint32_t G = perRegion ? 1u : (schedule.grid ? std::min(schedule.grid, resident_) : defaultGrid_);
   double total = 0.0;
-  for (const auto& w : work) total += std::max(w.cost, 0.f);
-  const double bal = schedule.balance > 0.f ? schedule.balance : 1.f;
+  uint64_t chunks = 0;
+  for (const auto& w : work) {
+    total += std::max(w.cost, 0.f);
+    chunks += std::max<uint32_t>(1, (w.samples + kChunk - 1) / kChunk);
+  }
+  uint32_t G = perRegion ? 1u : (schedule.grid ? std::min(schedule.grid, resident_) : defaultGrid_);
+  double bal = schedule.balance > 0.f ? schedule.balance : 1.f;
+  if (!perRegion && schedule.grid == 0) {
+    // The default grid leaves a third of the device to other streams' kernels
+    // (the next update's spatial phase).  That pays while the launch is one
+    // wave of teams; with more regions than workgroups, or many chunks for each,
+    // the launch is bound by throughput and takes most of the device: 1029 and
+    // 1957 regions of 700 samples 1.73 -> 1.58 and 0.73 -> 0.64 ms, 8 M samples
+    // in 363 regions 7.1 -> 4.9 ms (1 M samples in 48 to 150 regions: 0 to 5 %
+    // slower).  With many chunks per workgroup teams twice as large shorten the
+    // longest region, whose EM iterations are not known beforehand (10 M
+    // samples in two fields, two frames: 16.6 -> 15.7 ms; at two chunks per
+    // workgroup the smaller shares cost more than they give, 3.8 -> 4.0 ms).
+    if (work.size() > defaultGrid_ || chunks > kManyChunks * defaultGrid_)
+      G = std::max(defaultGrid_, resident_ - std::min(resident_, kLeaveGroups));
+    if (chunks > kManyChunks * defaultGrid_) bal *= 2.0;
+  }
   const double target = std::max(total / ((double)G * bal), 1e-30);
   const uint32_t minChunks = std::max<uint32_t>(1, schedule.minChunksPerRank);
   const uint32_t teamCap = std::max<uint32_t>(1, std::min(schedule.maxTeam, perRegionTeams ? resident_ : G));

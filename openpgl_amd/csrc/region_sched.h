@@ -16,7 +16,7 @@ struct DevBuf;
 // chunking and the fold order of the region kernel do not depend on them.
 struct RegionSchedule {
   int perRegionLaunches = 0;  // 1: one launch of one workgroup per region (plain per-region path)
-  uint32_t grid = 0;          // workgroups of the persistent launch (0: two per CU; at most all that fit at once)
+  uint32_t grid = 0;          // workgroups of the persistent launch (0: by the work, stage(); at most all that fit at once)
   float balance = 1.f;        // team target = total samples / (grid * balance), at least minChunksPerRank chunks
   uint32_t minChunksPerRank = 1;
   uint32_t maxTeam = 64;
