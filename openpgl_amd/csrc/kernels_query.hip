@@ -19,7 +19,64 @@
 
 namespace pglgpu {
 
-__device__ __forceinline__ int lookup_region(const QueryField& f, float x, float y, float z, float* u, uint32_t& id) {
+// The four lanes of a quad (lanes 4i .. 4i + 3 of a wave) work on one query:
+// lane q owns the components k = 4j + q (j < 8), so a query's component
+// loops take a quarter of the serial steps and the component parameters of
+// a region are read by four lanes at once.  Every lane of a quad runs the
+// same control flow (the query decides it), so the quad sums below see four
+// active lanes.
+//
+// Bound by the vector unit: the shift, product and pdf of a component are
+// about 150 instructions, most of them correctly rounded divisions and square
+// roots.  The component loops run over the groups that any query of the wave
+// uses, two groups per branch (a branch per component serialised their chains);
+// divisions by the same number share its reciprocal, and divisions and roots
+// whose operands are far from the ends of the exponent range go without the
+// scaling steps (2.07 M surface queries on 400 regions 466 -> 304 us).
+
+// DPP move inside a quad
+template <int CTRL>
+__device__ __forceinline__ uint32_t qdpp(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, true);
+}
+template <int CTRL>
+__device__ __forceinline__ float qdppf(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+
+// RegionNeighbours<8>::sampleApproximateClosestRegionIdx (spatial/KNN.h:134-148)
+// on a quad: lane q holds the keys of slots q and q + 4 (squared distance with
+// the slot in the low 3 bits, +inf for empty slots; keys are distinct, and as
+// unsigned integers in the order of the floats), ranks them among the eight,
+// and the slot of rank `sel` is the pick.
+__device__ __forceinline__ uint32_t quad_knn_pick(const QueryField& f, uint32_t leaf, int q, float x, float y, float z,
+                                                  float* u) {
+  const uint32_t sel = knn_draw(u, f.nbSize);
+  uint32_t id[2], key[2];
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const uint32_t s = (uint32_t)(q + 4 * h);
+    id[h] = f.nbIds[leaf * 8 + s];
+    const float4 p = f.nbPts[leaf * 8 + s];
+    const float d = knn_d2(p.x - x, p.y - y, p.z - z, f.knnFused != 0);
+    key[h] = ((id[h] == 0xffffffffu ? 0x7f800000u : __float_as_uint(d)) & ~7u) | s;
+  }
+  uint32_t rank[2] = {key[1] < key[0] ? 1u : 0u, key[0] < key[1] ? 1u : 0u};
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const uint32_t a = qdpp<0xB1>(key[h]), b = qdpp<0x4E>(key[h]), c = qdpp<0x1B>(key[h]);  // lanes q ^ 1, 2, 3
+#pragma unroll
+    for (int g = 0; g < 2; g++)
+      rank[g] += (a < key[g] ? 1u : 0u) + (b < key[g] ? 1u : 0u) + (c < key[g] ? 1u : 0u);
+  }
+  uint32_t r = (rank[0] == sel ? id[0] : 0u) | (rank[1] == sel ? id[1] : 0u);
+  r |= qdpp<0xB1>(r);
+  r |= qdpp<0x4E>(r);
+  return r;
+}
+
+__device__ __forceinline__ int lookup_region(const QueryField& f, int q, float x, float y, float z, float* u,
+                                             uint32_t& id) {
   if (!f.trained) return -1;
   if (!(x >= f.lo[0] && x <= f.hi[0] && y >= f.lo[1] && y <= f.hi[1] && z >= f.lo[2] && z <= f.hi[2])) return -1;
   uint32_t i = 0;
@@ -32,80 +89,152 @@ __device__ __forceinline__ int lookup_region(const QueryField& f, float x, float
   }
   const uint32_t leaf = nd.idx();
   id = leaf;
-  if (f.knn && *u >= 0.f) {
-    uint32_t ids[8];
-    float px[8], py[8], pz[8];
-    for (int s = 0; s < 8; s++) {
-      ids[s] = f.nbIds[leaf * 8 + s];
-      const float4 p = f.nbPts[leaf * 8 + s];
-      px[s] = p.x;
-      py[s] = p.y;
-      pz[s] = p.z;
-    }
-    return (int)knn_pick(ids, px, py, pz, f.nbSize, x, y, z, u, f.knnFused != 0);
-  }
+  if (f.knn && *u >= 0.f) return (int)quad_knn_pick(f, leaf, q, x, y, z, u);
   return (int)leaf;
 }
 
-// The four lanes of a quad (lanes 4i .. 4i + 3 of a wave) work on one query:
-// lane q owns the components k = 4j + q (j < 8), so a query's component
-// loops take a quarter of the serial steps and the component parameters of
-// a region are read by four lanes at once.  Every lane of a quad runs the
-// same control flow (the query decides it), so the quad sums below see four
-// active lanes.
-
 // sum over the quad; the same bits in its four lanes (IEEE addition commutes)
 __device__ __forceinline__ float qsum4(float v) {
-  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));  // lanes q ^ 1
-  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xF, 0xF, true));  // lanes q ^ 2
+  v += qdppf<0xB1>(v);  // lanes q ^ 1
+  v += qdppf<0x4E>(v);  // lanes q ^ 2
   return v;
 }
 
 // value of quad lane 0, 1, 2 or 3 (DPP quad broadcast)
 template <int L>
 __device__ __forceinline__ float qlane(float v) {
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), L * 0x55, 0xF, 0xF, false));
+  return qdppf<L * 0x55>(v);
+}
+
+// Correctly rounded n / d by the steps of the compiler's division (one
+// refinement of the reciprocal, two of the quotient), the reciprocal formed
+// once per d, without the scaling that only operands near the ends of the
+// exponent range need: the same quotient while d and n / d lie within
+// 2^-100 .. 2^100 (or n is 0).
+struct Recip {
+  float d, r;
+};
+__device__ __forceinline__ Recip recip_of(float d) {
+  const float r = __builtin_amdgcn_rcpf(d);
+  return {d, fmaf(fmaf(-d, r, 1.f), r, r)};
+}
+__device__ __forceinline__ float div_by(float n, const Recip& k) {
+  float q = n * k.r;
+  q = fmaf(fmaf(-k.d, q, n), k.r, q);
+  return fmaf(fmaf(-k.d, q, n), k.r, q);
+}
+
+// correctly rounded square root (x within 2^-90 .. 2^120, or 0): the nearest
+// of the hardware's estimate and its two neighbours
+__device__ __forceinline__ float sqrt_in_range(float x) {
+  const float s = __builtin_amdgcn_sqrtf(x);
+  const float dn = __int_as_float(__float_as_int(s) - 1), up = __int_as_float(__float_as_int(s) + 1);
+  const float ed = fmaf(-dn, s, x), eu = fmaf(-up, s, x);
+  const float r = ed <= 0.f ? dn : s;
+  return eu > 0.f ? up : r;
 }
 
 // This lane's components (k = 4j + q) after the parallax shift to the query
 // position: their directions, formed once per query and shared by every
-// product below.
+// product below.  Slots from K on hold a zero-weight component.
 struct LaneShift {
   float mx[8], my[8], mz[8];
 };
-__device__ __forceinline__ void lane_shift(const VMMParams& V, int q, bool par, float sx, float sy, float sz,
-                                           LaneShift& h) {
-  const int K = V.K;
+
+__device__ __forceinline__ void lane_shift(const VMMParams& V, int k, bool par, float sx, float sy, float sz, float& mx,
+                                           float& my, float& mz) {
+  mx = V.mux[k];
+  my = V.muy[k];
+  mz = V.muz[k];
+  if (par) {  // shift_comp
+    const float d = V.dist[k];
+    const float px = fmaf(mx, d, sx), py = fmaf(my, d, sy), pz = fmaf(mz, d, sz);
+    const float l = sqrt_in_range(qdot(px, py, pz, px, py, pz));
+    const Recip rl = recip_of(l);
+    float qx = div_by(px, rl), qy = div_by(py, rl), qz = div_by(pz, rl);
+    // a distance whose square leaves the exponent range (a component may carry any)
+    if (__ballot(!(l > 1e-15f && l < 1e18f)) != 0) {
+      qx = px / l;
+      qy = py / l;
+      qz = pz / l;
+    }
+    const bool shift = d > 0.f && isfinite(d);
+    mx = shift ? qx : mx;
+    my = shift ? qy : my;
+    mz = shift ? qz : mz;
+  }
+}
+
+// Product of one shifted component with the lobe (weight, n, kn, nn):
+// product_comp of query_math.h with shared reciprocals and every fused
+// multiply-add written out (each use of it rounds alike).
+__device__ __forceinline__ ProdComp lane_product(float w, float kappa, float mx, float my, float mz, float norm,
+                                                 float weight, float nx, float ny, float nz, float kn, float nn) {
+  ProdComp p;
+  float ax = fmaf(kappa, mx, kn * nx), ay = fmaf(kappa, my, kn * ny), az = fmaf(kappa, mz, kn * nz);
+  float nk = sqrt_in_range(qdot(ax, ay, az, ax, ay, az));
+  const bool ok = nk > 1e-3f;
+  nk = ok ? nk : 0.f;
+  const Recip k = recip_of(nk);
+  ax = ok ? div_by(ax, k) : mx;
+  ay = ok ? div_by(ay, k) : my;
+  az = ok ? div_by(az, k) : mz;
+  const float e = expf(-2.f * nk);
+  float nrm = div_by(nk, recip_of(2.f * 3.14159265358979f * (1.f - e)));
+  nrm = ok ? nrm : kOneOverFourPi;
+  float scale = div_by(norm * nn, recip_of(nrm));
+  const float c0 = qdot(mx, my, mz, ax, ay, az);
+  const float c1 = qdot(nx, ny, nz, ax, ay, az);
+  scale *= expf(fmaf(kappa, c0 - 1.f, kn * (c1 - 1.f)));
+  scale *= w * weight;
+  p.scale = scale;
+  p.kappa = nk;
+  p.mx = ax;
+  p.my = ay;
+  p.mz = az;
+  p.norm = nrm;
+  p.em2k = e;
+  return p;
+}
+
+// part + eval_comp(...)
+__device__ __forceinline__ float eval_add(float part, float w, float norm, float kappa, float mx, float my, float mz,
+                                          float dx, float dy, float dz) {
+  const float c = qdot(dx, dy, dz, mx, my, mz);
+  return fmaf(norm * expf(kappa * fminf(c - 1.f, 0.f)), w, part);
+}
+
+// Calls f(j) for the component groups j < J (J uniform over the wave), two
+// groups per branch.
+template <class F>
+__device__ __forceinline__ void for_groups(int J, F&& f) {
 #pragma unroll
-  for (int j = 0; j < 8; j++) {
-    const int k = 4 * j + q;
-    h.mx[j] = 0.f; h.my[j] = 0.f; h.mz[j] = 1.f;
-    if (k < K) {
-      float d;
-      shift_comp(V, k, sx, sy, sz, h.mx[j], h.my[j], h.mz[j], d, par);
+  for (int j = 0; j < 8; j += 2) {
+    if (j < J) {
+      f(j);
+      f(j + 1);
     }
   }
 }
 
-// Products of this lane's shifted components with the lobe (weight, n, kn,
-// nn): scale 0 for k >= K.
+// Products of this lane's components with a lobe: scale 0 for k >= K.
 struct LaneComps {
   float s[8], kap[8], mx[8], my[8], mz[8], nrm[8], e2k[8];
 };
-__device__ __forceinline__ void lane_products(const VMMParams& V, int q, const LaneShift& h, float weight, float nx,
-                                              float ny, float nz, float kn, float nn, LaneComps& c) {
+__device__ __forceinline__ void lane_products(const VMMParams& V, int q, int J, const LaneShift& h, float weight,
+                                              float nx, float ny, float nz, float kn, float nn, LaneComps& c) {
   const int K = V.K;
 #pragma unroll
   for (int j = 0; j < 8; j++) {
-    const int k = 4 * j + q;
     c.s[j] = 0.f; c.kap[j] = 0.f; c.mx[j] = 0.f; c.my[j] = 0.f; c.mz[j] = 1.f; c.nrm[j] = 0.f; c.e2k[j] = 1.f;
-    if (k < K) {
-      const ProdComp p =
-          product_comp(V.w[k], V.kappa[k], h.mx[j], h.my[j], h.mz[j], V.norm[k], weight, nx, ny, nz, kn, nn);
-      c.s[j] = p.scale; c.kap[j] = p.kappa; c.mx[j] = p.mx; c.my[j] = p.my; c.mz[j] = p.mz; c.nrm[j] = p.norm;
-      c.e2k[j] = p.em2k;
-    }
   }
+  for_groups(J, [&](int j) {
+    const int k = 4 * j + q;
+    const ProdComp p =
+        lane_product(V.w[k], V.kappa[k], h.mx[j], h.my[j], h.mz[j], V.norm[k], weight, nx, ny, nz, kn, nn);
+    c.s[j] = k < K ? p.scale : 0.f; c.kap[j] = p.kappa; c.mx[j] = p.mx; c.my[j] = p.my; c.mz[j] = p.mz;
+    c.nrm[j] = p.norm; c.e2k[j] = p.em2k;
+  });
 }
 
 // integral of the product of the shifted mixture with the lobe (quad sum)
@@ -117,31 +246,32 @@ __device__ __forceinline__ float quad_integral(const LaneComps& c) {
 }
 
 // pdf at direction d of the product held in c (quad sum)
-__device__ __forceinline__ float quad_pdf(const VMMParams& V, int q, const LaneComps& c, float integral, float dx,
-                                          float dy, float dz) {
+__device__ __forceinline__ float quad_pdf(const VMMParams& V, int q, int J, const LaneComps& c, float integral,
+                                          float dx, float dy, float dz) {
   const float inv = 1.f / integral;
+  const int K = V.K;
   float part = 0.f;
-#pragma unroll
-  for (int j = 0; j < 8; j++)
-    if (4 * j + q < V.K) part += eval_comp(c.s[j] * inv, c.nrm[j], c.kap[j], c.mx[j], c.my[j], c.mz[j], dx, dy, dz);
+  for_groups(J, [&](int j) {
+    const float v = eval_add(part, c.s[j] * inv, c.nrm[j], c.kap[j], c.mx[j], c.my[j], c.mz[j], dx, dy, dz);
+    part = 4 * j + q < K ? v : part;
+  });
   return qsum4(part);
 }
 
 // pdf at d of the product with a lobe, the products formed on the fly (quad sum)
-__device__ __forceinline__ float quad_pdf_lobe(const VMMParams& V, int q, const LaneShift& h, float weight, float nx,
-                                               float ny, float nz, float kn, float nn, float integral, float dx,
-                                               float dy, float dz) {
+__device__ __forceinline__ float quad_pdf_lobe(const VMMParams& V, int q, int J, const LaneShift& h, float weight,
+                                               float nx, float ny, float nz, float kn, float nn, float integral,
+                                               float dx, float dy, float dz) {
   const float inv = 1.f / integral;
+  const int K = V.K;
   float part = 0.f;
-#pragma unroll
-  for (int j = 0; j < 8; j++) {
+  for_groups(J, [&](int j) {
     const int k = 4 * j + q;
-    if (k < V.K) {
-      const ProdComp p =
-          product_comp(V.w[k], V.kappa[k], h.mx[j], h.my[j], h.mz[j], V.norm[k], weight, nx, ny, nz, kn, nn);
-      part += eval_comp(p.scale * inv, p.norm, p.kappa, p.mx, p.my, p.mz, dx, dy, dz);
-    }
-  }
+    const ProdComp p =
+        lane_product(V.w[k], V.kappa[k], h.mx[j], h.my[j], h.mz[j], V.norm[k], weight, nx, ny, nz, kn, nn);
+    const float v = eval_add(part, p.scale * inv, p.norm, p.kappa, p.mx, p.my, p.mz, dx, dy, dz);
+    part = k < K ? v : part;
+  });
   return qsum4(part);
 }
 
@@ -150,32 +280,33 @@ __device__ __forceinline__ float quad_pdf_lobe(const VMMParams& V, int q, const 
 // reaches u1 (the last one if rounding leaves the total short), then u0 and
 // the rescaled u1 sample it.  The walk goes over groups of four components
 // (one per lane) and then inside the chosen group.
-__device__ __forceinline__ void quad_sample(const VMMParams& V, int q, int lane, const LaneComps& c, float integral,
-                                            float u0, float u1, float* out) {
+__device__ __forceinline__ void quad_sample(const VMMParams& V, int q, int lane, int Jw, const LaneComps& c,
+                                            float integral, float u0, float u1, float* out) {
   const int K = V.K;
   const int J = (K + 3) >> 2;
-  float acc = 0.f, accs = 0.f;  // share of the groups before group js
+  // an integral near the ends of the exponent range needs the scaled division
+  const bool plain = __ballot(!(integral > 1e-20f && integral < 1e20f)) == 0;
+  const Recip ri = recip_of(integral);
+  float acc = 0.f, accs = 0.f;  // share of the groups before the chosen one
   int js = -1;
-#pragma unroll
-  for (int j = 0; j < 8; j++) {
-    if (j < J && js < 0) {
-      const float g = qsum4(c.s[j] / integral);
-      if (acc + g >= u1 || j == J - 1) {  // the last group is walked in any case
-        js = j;
-        accs = acc;
-      } else {
-        acc += g;
-      }
-    }
-  }
-  // this lane's share in group js and the values of its component
+  // this lane's share in the chosen group and the values of its component
   float x = 0.f, kap = 0.f, e2k = 1.f, mx = 0.f, my = 0.f, mz = 1.f;
-#pragma unroll
-  for (int j = 0; j < 8; j++) {
-    if (j == js) {
-      x = c.s[j] / integral; kap = c.kap[j]; e2k = c.e2k[j]; mx = c.mx[j]; my = c.my[j]; mz = c.mz[j];
-    }
-  }
+  for_groups(Jw, [&](int j) {
+    float sh = div_by(c.s[j], ri);
+    if (!plain) sh = c.s[j] / integral;
+    const float g = qsum4(sh);
+    const bool open = js < 0 && j < J;
+    const bool take = open && (acc + g >= u1 || j == J - 1);  // the last group is walked in any case
+    js = take ? j : js;
+    accs = take ? acc : accs;
+    x = take ? sh : x;
+    kap = take ? c.kap[j] : kap;
+    e2k = take ? c.e2k[j] : e2k;
+    mx = take ? c.mx[j] : mx;
+    my = take ? c.my[j] : my;
+    mz = take ? c.mz[j] : mz;
+    acc = open ? acc + g : acc;
+  });
   const float x0 = qlane<0>(x), x1 = qlane<1>(x), x2 = qlane<2>(x), x3 = qlane<3>(x);
   const int last = 4 * js + 3 < K ? 3 : ((K - 1) & 3);  // last component of the group
   // the walk inside the group: components 4 js + l, l = 0 .. last
@@ -202,6 +333,13 @@ __device__ __forceinline__ void quad_sample(const VMMParams& V, int q, int lane,
   sample_comp(kap, e2k, mx, my, mz, u0, us, out);
 }
 
+// largest component group count of the wave's active lanes
+__device__ __forceinline__ int wave_groups(int K) {
+  int J = 8;
+  while (J > 1 && __ballot(K > 4 * (J - 1)) == 0) J--;
+  return J;
+}
+
 // One query on the four lanes of a quad: lookup (+ KNN pick), parallax shift,
 // cosine (surface) or 3-lobe HG (volume) product, one sample and its pdf.
 // Invalid queries (outside the field, untrained field, invalid region) give
@@ -216,7 +354,7 @@ __device__ __forceinline__ void query_quad(const QueryField& surf, const QueryFi
   pdf = 0.f;
   integral = 0.f;
   out[0] = out[1] = out[2] = 0.f;
-  const int r = lookup_region(f, x, y, z, &u, id);
+  const int r = lookup_region(f, q, x, y, z, &u, id);
   if (r < 0 || !f.regions[r].valid) {
     id = 0xffffffffu;
     return;
@@ -224,15 +362,16 @@ __device__ __forceinline__ void query_quad(const QueryField& surf, const QueryFi
   const VMMParams& V = f.regions[r].vmm;
   const bool par = f.parallax != 0;
   const float sx = V.pivot[0] - x, sy = V.pivot[1] - y, sz = V.pivot[2] - z;
+  const int J = wave_groups(V.K);
   LaneShift h;
-  lane_shift(V, q, par, sx, sy, sz, h);
+  for_groups(J, [&](int j) { lane_shift(V, 4 * j + q, par, sx, sy, sz, h.mx[j], h.my[j], h.mz[j]); });
   LaneComps c;
   if (!volume) {
     const float kn = kCosineKappa, nn = cosine_normalization();
-    lane_products(V, q, h, 1.f, nx, ny, nz, kn, nn, c);
+    lane_products(V, q, J, h, 1.f, nx, ny, nz, kn, nn, c);
     integral = quad_integral(c);
-    quad_sample(V, q, lane, c, integral, ux, uy, out);
-    pdf = quad_pdf(V, q, c, integral, out[0], out[1], out[2]);
+    quad_sample(V, q, lane, J, c, integral, ux, uy, out);
+    pdf = quad_pdf(V, q, J, c, integral, out[0], out[1], out[2]);
   } else {
     const HGRep& rep = hg[hg_index(g)];
     const int KP = (int)rep.K;
@@ -240,7 +379,7 @@ __device__ __forceinline__ void query_quad(const QueryField& surf, const QueryFi
     float sum = 0.f;
     for (int m = 0; m < KP; m++) {
       sgn[m] = (g * rep.mc[m] > 0.f) ? 1.f : -1.f;
-      lane_products(V, q, h, rep.w[m], nx * sgn[m], ny * sgn[m], nz * sgn[m], rep.kappa[m], rep.norm[m], c);
+      lane_products(V, q, J, h, rep.w[m], nx * sgn[m], ny * sgn[m], nz * sgn[m], rep.kappa[m], rep.norm[m], c);
       integ[m] = quad_integral(c);
       sum += integ[m];
     }
@@ -253,12 +392,11 @@ __device__ __forceinline__ void query_quad(const QueryField& surf, const QueryFi
       if (nw > ux) break;
       acc = nw;
     }
-    lane_products(V, q, h, rep.w[m], nx * sgn[m], ny * sgn[m], nz * sgn[m], rep.kappa[m], rep.norm[m], c);
-    quad_sample(V, q, lane, c, integ[m], (ux - acc) / mw[m], uy, out);
+    lane_products(V, q, J, h, rep.w[m], nx * sgn[m], ny * sgn[m], nz * sgn[m], rep.kappa[m], rep.norm[m], c);
+    quad_sample(V, q, lane, J, c, integ[m], (ux - acc) / mw[m], uy, out);
     for (int j = 0; j < KP; j++)
-      pdf += mw[j] * (j == m ? quad_pdf(V, q, c, integ[j], out[0], out[1], out[2])
-                             : quad_pdf_lobe(V, q, h, rep.w[j], nx * sgn[j], ny * sgn[j], nz * sgn[j], rep.kappa[j],
-                                             rep.norm[j], integ[j], out[0], out[1], out[2]));
+      pdf += mw[j] * quad_pdf_lobe(V, q, J, h, rep.w[j], nx * sgn[j], ny * sgn[j], nz * sgn[j], rep.kappa[j],
+                                   rep.norm[j], integ[j], out[0], out[1], out[2]);
     integral = sum;
   }
 }
