@@ -136,8 +136,18 @@ struct RegionState {
   // counts: [7] team size, [8] E-step passes, [11] samples
   float prof[12];
   int32_t initK;        // components of the initial mixture of a fit (0: the factory's initK)
-  uint32_t pad[304];
+  // the mixture as the query kernel reads it, component by component: a quad
+  // of lanes reads four components' halves as one 64-byte line
+  struct alignas(16) QueryComp {
+    float mux, muy, muz, dist, w, kappa, norm, unused;
+  } query[32];
+  uint32_t pad[48];
 };
+// component k of the mixture into its query form (whoever writes a state does this for all 32)
+PGL_HD inline void pack_query_comp(RegionState& S, int k) {
+  const VMMParams& V = S.vmm;
+  S.query[k] = RegionState::QueryComp{V.mux[k], V.muy[k], V.muz[k], V.dist[k], V.w[k], V.kappa[k], V.norm[k], 0.f};
+}
 static_assert(sizeof(RegionState) == 4096, "RegionState must be 4 KiB");
 
 // Integer sample statistics accumulator of one kd node (data/SampleStatistics.h:195-342)

@@ -396,6 +396,8 @@ void KindField::readFile(std::istream& is, int W, bool parallaxAware, hipStream_
 
   if (R > 0) {
     ensureRegionCapacity(R, s);
+    for (auto& st : states)
+      for (int k = 0; k < 32; k++) pack_query_comp(st, k);
     PGL_HIP_CHECK(hipMemcpyAsync(dStates_.p, states.data(), size_t(R) * sizeof(RegionState), hipMemcpyHostToDevice, s));
   }
   if (N > 0) {

@@ -152,8 +152,9 @@ struct QueryPiece {
   uint32_t* id;
   uint32_t begin, n;
 };
+// volumes: some piece has a vol array
 void launch_query_pieces(const QueryField& surf, const QueryField& vol, const HGRep* hg, const QueryPiece* pieces,
-                         uint32_t numPieces, uint32_t n, hipStream_t s);
+                         uint32_t numPieces, uint32_t n, bool volumes, hipStream_t s);
 void launch_query(const QueryField& surf, const QueryField& vol, const HGRep* hg, uint32_t n, const float* pos,
                   const float* nrm, const float* g, const float* u2, const float* u1, const uint8_t* isVolume,
                   float* dirOut, float* pdfOut, uint32_t* idOut, float* integralOut, hipStream_t s);

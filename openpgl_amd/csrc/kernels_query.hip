@@ -32,7 +32,11 @@ namespace pglgpu {
 // uses, two groups per branch (a branch per component serialised their chains);
 // divisions by the same number share its reciprocal, and divisions and roots
 // whose operands are far from the ends of the exponent range go without the
-// scaling steps (2.07 M surface queries on 400 regions 466 -> 304 us).
+// scaling steps.  A component is read as two 16-byte loads of its region's
+// query form (seven loads of one word each, from as many cache lines, took as
+// long as the arithmetic).  2.07 M surface queries on 400 regions: 463 us at
+// first, 378 with the arithmetic above, 320 at five instead of three waves per
+// SIMD, 261 with the query form.
 
 // DPP move inside a quad
 template <int CTRL>
@@ -141,13 +145,23 @@ struct LaneShift {
   float mx[8], my[8], mz[8];
 };
 
-__device__ __forceinline__ void lane_shift(const VMMParams& V, int k, bool par, float sx, float sy, float sz, float& mx,
+// A region's components as 16-byte halves: direction and distance, then weight,
+// concentration and normalisation (RegionState::QueryComp).
+struct Mixture {
+  const float4* q;
+  int K;
+  __device__ __forceinline__ float4 dir(int k) const { return q[2 * k]; }
+  __device__ __forceinline__ float4 lobe(int k) const { return q[2 * k + 1]; }
+};
+
+__device__ __forceinline__ void lane_shift(const Mixture& V, int k, bool par, float sx, float sy, float sz, float& mx,
                                            float& my, float& mz) {
-  mx = V.mux[k];
-  my = V.muy[k];
-  mz = V.muz[k];
+  const float4 a = V.dir(k);
+  mx = a.x;
+  my = a.y;
+  mz = a.z;
   if (par) {  // shift_comp
-    const float d = V.dist[k];
+    const float d = a.w;
     const float px = fmaf(mx, d, sx), py = fmaf(my, d, sy), pz = fmaf(mz, d, sz);
     const float l = sqrt_in_range(qdot(px, py, pz, px, py, pz));
     const Recip rl = recip_of(l);
@@ -168,8 +182,9 @@ __device__ __forceinline__ void lane_shift(const VMMParams& V, int k, bool par, 
 // Product of one shifted component with the lobe (weight, n, kn, nn):
 // product_comp of query_math.h with shared reciprocals and every fused
 // multiply-add written out (each use of it rounds alike).
-__device__ __forceinline__ ProdComp lane_product(float w, float kappa, float mx, float my, float mz, float norm,
-                                                 float weight, float nx, float ny, float nz, float kn, float nn) {
+__device__ __forceinline__ ProdComp lane_product(const float4 b, float mx, float my, float mz, float weight,
+                                                 float nx, float ny, float nz, float kn, float nn) {
+  const float w = b.x, kappa = b.y, norm = b.z;
   ProdComp p;
   float ax = fmaf(kappa, mx, kn * nx), ay = fmaf(kappa, my, kn * ny), az = fmaf(kappa, mz, kn * nz);
   float nk = sqrt_in_range(qdot(ax, ay, az, ax, ay, az));
@@ -217,36 +232,14 @@ __device__ __forceinline__ void for_groups(int J, F&& f) {
   }
 }
 
-// Products of this lane's components with a lobe: scale 0 for k >= K.
+// Products of this lane's shifted components with the cosine lobe, held from
+// the integral to the pdf: scale 0 for k >= K.
 struct LaneComps {
-  float s[8], kap[8], mx[8], my[8], mz[8], nrm[8], e2k[8];
+  float s[8], kap[8], mx[8], my[8], mz[8], nrm[8];
 };
-__device__ __forceinline__ void lane_products(const VMMParams& V, int q, int J, const LaneShift& h, float weight,
-                                              float nx, float ny, float nz, float kn, float nn, LaneComps& c) {
-  const int K = V.K;
-#pragma unroll
-  for (int j = 0; j < 8; j++) {
-    c.s[j] = 0.f; c.kap[j] = 0.f; c.mx[j] = 0.f; c.my[j] = 0.f; c.mz[j] = 1.f; c.nrm[j] = 0.f; c.e2k[j] = 1.f;
-  }
-  for_groups(J, [&](int j) {
-    const int k = 4 * j + q;
-    const ProdComp p =
-        lane_product(V.w[k], V.kappa[k], h.mx[j], h.my[j], h.mz[j], V.norm[k], weight, nx, ny, nz, kn, nn);
-    c.s[j] = k < K ? p.scale : 0.f; c.kap[j] = p.kappa; c.mx[j] = p.mx; c.my[j] = p.my; c.mz[j] = p.mz;
-    c.nrm[j] = p.norm; c.e2k[j] = p.em2k;
-  });
-}
-
-// integral of the product of the shifted mixture with the lobe (quad sum)
-__device__ __forceinline__ float quad_integral(const LaneComps& c) {
-  float part = 0.f;
-#pragma unroll
-  for (int j = 0; j < 8; j++) part += c.s[j];
-  return qsum4(part);
-}
 
 // pdf at direction d of the product held in c (quad sum)
-__device__ __forceinline__ float quad_pdf(const VMMParams& V, int q, int J, const LaneComps& c, float integral,
+__device__ __forceinline__ float quad_pdf(const Mixture& V, int q, int J, const LaneComps& c, float integral,
                                           float dx, float dy, float dz) {
   const float inv = 1.f / integral;
   const int K = V.K;
@@ -259,7 +252,7 @@ __device__ __forceinline__ float quad_pdf(const VMMParams& V, int q, int J, cons
 }
 
 // pdf at d of the product with a lobe, the products formed on the fly (quad sum)
-__device__ __forceinline__ float quad_pdf_lobe(const VMMParams& V, int q, int J, const LaneShift& h, float weight,
+__device__ __forceinline__ float quad_pdf_lobe(const Mixture& V, int q, int J, const LaneShift& h, float weight,
                                                float nx, float ny, float nz, float kn, float nn, float integral,
                                                float dx, float dy, float dz) {
   const float inv = 1.f / integral;
@@ -268,43 +261,52 @@ __device__ __forceinline__ float quad_pdf_lobe(const VMMParams& V, int q, int J,
   for_groups(J, [&](int j) {
     const int k = 4 * j + q;
     const ProdComp p =
-        lane_product(V.w[k], V.kappa[k], h.mx[j], h.my[j], h.mz[j], V.norm[k], weight, nx, ny, nz, kn, nn);
+        lane_product(V.lobe(k), h.mx[j], h.my[j], h.mz[j], weight, nx, ny, nz, kn, nn);
     const float v = eval_add(part, p.scale * inv, p.norm, p.kappa, p.mx, p.my, p.mz, dx, dy, dz);
     part = k < K ? v : part;
   });
   return qsum4(part);
 }
 
-// One direction from the product held in c (PAVMM::sample): the component is
-// the first k, in component order, whose cumulative share of the integral
-// reaches u1 (the last one if rounding leaves the total short), then u0 and
-// the rescaled u1 sample it.  The walk goes over groups of four components
-// (one per lane) and then inside the chosen group.
-__device__ __forceinline__ void quad_sample(const VMMParams& V, int q, int lane, int Jw, const LaneComps& c,
-                                            float integral, float u0, float u1, float* out) {
+// sum of this lane's product weights over the quad
+__device__ __forceinline__ float quad_integral(const float s[8]) {
+  float part = 0.f;
+#pragma unroll
+  for (int j = 0; j < 8; j++) part += s[j];
+  return qsum4(part);
+}
+
+// The component PAVMM::sample takes for u1: the first k, in component order,
+// whose cumulative share of the integral reaches u1 (the last one if rounding
+// leaves the total short).  The walk goes over groups of four components (one
+// per lane; `group(j)` is called for every group until it is found, with
+// whether it is the one) and then inside the chosen group.  u1 is rescaled to
+// the component's share.
+struct Pick {
+  int js, qs;  // component 4 js + qs
+  float us;
+};
+template <class F>
+__device__ __forceinline__ Pick quad_pick(const Mixture& V, int Jw, const float s[8], float integral, float u1,
+                                          F&& group) {
   const int K = V.K;
   const int J = (K + 3) >> 2;
   // an integral near the ends of the exponent range needs the scaled division
   const bool plain = __ballot(!(integral > 1e-20f && integral < 1e20f)) == 0;
   const Recip ri = recip_of(integral);
   float acc = 0.f, accs = 0.f;  // share of the groups before the chosen one
+  float x = 0.f;                // this lane's share in the chosen group
   int js = -1;
-  // this lane's share in the chosen group and the values of its component
-  float x = 0.f, kap = 0.f, e2k = 1.f, mx = 0.f, my = 0.f, mz = 1.f;
   for_groups(Jw, [&](int j) {
-    float sh = div_by(c.s[j], ri);
-    if (!plain) sh = c.s[j] / integral;
+    float sh = div_by(s[j], ri);
+    if (!plain) sh = s[j] / integral;
     const float g = qsum4(sh);
     const bool open = js < 0 && j < J;
     const bool take = open && (acc + g >= u1 || j == J - 1);  // the last group is walked in any case
     js = take ? j : js;
     accs = take ? acc : accs;
     x = take ? sh : x;
-    kap = take ? c.kap[j] : kap;
-    e2k = take ? c.e2k[j] : e2k;
-    mx = take ? c.mx[j] : mx;
-    my = take ? c.my[j] : my;
-    mz = take ? c.mz[j] : mz;
+    group(j, take);
     acc = open ? acc + g : acc;
   });
   const float x0 = qlane<0>(x), x1 = qlane<1>(x), x2 = qlane<2>(x), x3 = qlane<3>(x);
@@ -323,14 +325,7 @@ __device__ __forceinline__ void quad_sample(const VMMParams& V, int q, int lane,
     }
   }
   const float cdf = qs == 0 ? x0 : (qs == 1 ? x1 : (qs == 2 ? x2 : x3));
-  const int src = (lane & ~3) | qs;
-  kap = __shfl(kap, src);
-  e2k = __shfl(e2k, src);
-  mx = __shfl(mx, src);
-  my = __shfl(my, src);
-  mz = __shfl(mz, src);
-  const float us = fminf(1.f - 1.19209290e-7f, (u1 - sum) / cdf);
-  sample_comp(kap, e2k, mx, my, mz, u0, us, out);
+  return {js, qs, fminf(1.f - 1.19209290e-7f, (u1 - sum) / cdf)};
 }
 
 // largest component group count of the wave's active lanes
@@ -343,12 +338,15 @@ __device__ __forceinline__ int wave_groups(int K) {
 // One query on the four lanes of a quad: lookup (+ KNN pick), parallax shift,
 // cosine (surface) or 3-lobe HG (volume) product, one sample and its pdf.
 // Invalid queries (outside the field, untrained field, invalid region) give
-// dir 0, pdf 0, id ~0.  Every lane returns the same results.
+// dir 0, pdf 0, id ~0.  Every lane returns the same results.  VOLUMES: the
+// batch may hold volume queries (their registers are most of the kernel's: a
+// batch of surface queries alone runs five waves to a SIMD, with them four).
+template <bool VOLUMES>
 __device__ __forceinline__ void query_quad(const QueryField& surf, const QueryField& vol, const HGRep* __restrict__ hg,
                                            bool volume, float x, float y, float z, float nx, float ny, float nz,
                                            float g, float ux, float uy, float u, float out[3], float& pdf,
                                            uint32_t& id, float& integral) {
-  const QueryField& f = volume ? vol : surf;
+  const QueryField& f = VOLUMES && volume ? vol : surf;
   const int lane = threadIdx.x & 63, q = lane & 3;
   id = 0xffffffffu;
   pdf = 0.f;
@@ -359,49 +357,112 @@ __device__ __forceinline__ void query_quad(const QueryField& surf, const QueryFi
     id = 0xffffffffu;
     return;
   }
-  const VMMParams& V = f.regions[r].vmm;
+  const RegionState& S = f.regions[r];
+  const Mixture V{(const float4*)S.query, S.vmm.K};
   const bool par = f.parallax != 0;
-  const float sx = V.pivot[0] - x, sy = V.pivot[1] - y, sz = V.pivot[2] - z;
-  const int J = wave_groups(V.K);
-  LaneShift h;
-  for_groups(J, [&](int j) { lane_shift(V, 4 * j + q, par, sx, sy, sz, h.mx[j], h.my[j], h.mz[j]); });
-  LaneComps c;
-  if (!volume) {
+  const float sx = S.vmm.pivot[0] - x, sy = S.vmm.pivot[1] - y, sz = S.vmm.pivot[2] - z;
+  const int K = V.K;
+  const int J = wave_groups(K);
+  if (!VOLUMES || !volume) {
     const float kn = kCosineKappa, nn = cosine_normalization();
-    lane_products(V, q, J, h, 1.f, nx, ny, nz, kn, nn, c);
-    integral = quad_integral(c);
-    quad_sample(V, q, lane, J, c, integral, ux, uy, out);
+    LaneComps c;
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      c.s[j] = 0.f; c.kap[j] = 0.f; c.mx[j] = 0.f; c.my[j] = 0.f; c.mz[j] = 1.f; c.nrm[j] = 0.f;
+    }
+    for_groups(J, [&](int j) {
+      const int k = 4 * j + q;
+      float hx, hy, hz;
+      lane_shift(V, k, par, sx, sy, sz, hx, hy, hz);
+      const ProdComp p = lane_product(V.lobe(k), hx, hy, hz, 1.f, nx, ny, nz, kn, nn);
+      c.s[j] = k < K ? p.scale : 0.f; c.kap[j] = p.kappa; c.mx[j] = p.mx; c.my[j] = p.my; c.mz[j] = p.mz;
+      c.nrm[j] = p.norm;
+    });
+    integral = quad_integral(c.s);
+    float kap = 0.f, mx = 0.f, my = 0.f, mz = 1.f;  // of this lane's component in the chosen group
+    const Pick pk = quad_pick(V, J, c.s, integral, uy, [&](int j, bool take) {
+      kap = take ? c.kap[j] : kap;
+      mx = take ? c.mx[j] : mx;
+      my = take ? c.my[j] : my;
+      mz = take ? c.mz[j] : mz;
+    });
+    const int src = (lane & ~3) | pk.qs;
+    kap = __shfl(kap, src);
+    sample_comp(kap, expf(-2.f * kap), __shfl(mx, src), __shfl(my, src), __shfl(mz, src), ux, pk.us, out);
     pdf = quad_pdf(V, q, J, c, integral, out[0], out[1], out[2]);
   } else {
     const HGRep& rep = hg[hg_index(g)];
     const int KP = (int)rep.K;
-    float integ[4], sgn[4];
+    LaneShift h;
+    for_groups(J, [&](int j) { lane_shift(V, 4 * j + q, par, sx, sy, sz, h.mx[j], h.my[j], h.mz[j]); });
+    // the product weights of every lobe are kept; of the products themselves
+    // only the sampled component's is formed again
+    float s[4][8], integ[4], mw[4], sgn[4];
     float sum = 0.f;
-    for (int m = 0; m < KP; m++) {
-      sgn[m] = (g * rep.mc[m] > 0.f) ? 1.f : -1.f;
-      lane_products(V, q, J, h, rep.w[m], nx * sgn[m], ny * sgn[m], nz * sgn[m], rep.kappa[m], rep.norm[m], c);
-      integ[m] = quad_integral(c);
-      sum += integ[m];
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+#pragma unroll
+      for (int j = 0; j < 8; j++) s[m][j] = 0.f;
+      integ[m] = 0.f;
+      sgn[m] = 1.f;
+      if (__ballot(m < KP) != 0) {
+        sgn[m] = (g * rep.mc[m] > 0.f) ? 1.f : -1.f;
+        const float weight = rep.w[m], kn = rep.kappa[m], nn = rep.norm[m];
+        for_groups(J, [&](int j) {
+          const int k = 4 * j + q;
+          const ProdComp p = lane_product(V.lobe(k), h.mx[j], h.my[j], h.mz[j], weight,
+                                          nx * sgn[m], ny * sgn[m], nz * sgn[m], kn, nn);
+          s[m][j] = k < K ? p.scale : 0.f;
+        });
+        integ[m] = quad_integral(s[m]);
+        sum = m < KP ? sum + integ[m] : sum;
+      }
     }
-    float mw[4];
-    for (int m = 0; m < KP; m++) mw[m] = integ[m] / sum;
+#pragma unroll
+    for (int m = 0; m < 4; m++) mw[m] = integ[m] / sum;
+    // the lobe: the first whose cumulative share exceeds ux (the last one in any case)
     float acc = 0.f;
-    int m = 0;
-    for (; m < KP - 1; ++m) {
+    int lobe = 0;
+    bool open = true;
+#pragma unroll
+    for (int m = 0; m < 3; m++) {
       const float nw = acc + mw[m];
-      if (nw > ux) break;
-      acc = nw;
+      open = open && m < KP - 1 && !(nw > ux);
+      acc = open ? nw : acc;
+      lobe = open ? m + 1 : lobe;
     }
-    lane_products(V, q, J, h, rep.w[m], nx * sgn[m], ny * sgn[m], nz * sgn[m], rep.kappa[m], rep.norm[m], c);
-    quad_sample(V, q, lane, J, c, integ[m], (ux - acc) / mw[m], uy, out);
-    for (int j = 0; j < KP; j++)
-      pdf += mw[j] * quad_pdf_lobe(V, q, J, h, rep.w[j], nx * sgn[j], ny * sgn[j], nz * sgn[j], rep.kappa[j],
-                                   rep.norm[j], integ[j], out[0], out[1], out[2]);
+    float sl[8], integral1 = integ[0], w1 = mw[0], sg = sgn[0];
+#pragma unroll
+    for (int j = 0; j < 8; j++) sl[j] = s[0][j];
+#pragma unroll
+    for (int m = 1; m < 4; m++) {
+      const bool it = lobe == m;
+      integral1 = it ? integ[m] : integral1;
+      w1 = it ? mw[m] : w1;
+      sg = it ? sgn[m] : sg;
+#pragma unroll
+      for (int j = 0; j < 8; j++) sl[j] = it ? s[m][j] : sl[j];
+    }
+    const Pick pk = quad_pick(V, J, sl, integral1, uy, [](int, bool) {});
+    const int k = 4 * pk.js + pk.qs;
+    float hx, hy, hz;
+    lane_shift(V, k, par, sx, sy, sz, hx, hy, hz);
+    const ProdComp p = lane_product(V.lobe(k), hx, hy, hz, rep.w[lobe], nx * sg, ny * sg, nz * sg,
+                                    rep.kappa[lobe], rep.norm[lobe]);
+    sample_comp(p.kappa, p.em2k, p.mx, p.my, p.mz, (ux - acc) / w1, pk.us, out);
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+      if (__ballot(m < KP) == 0) continue;
+      const float v = quad_pdf_lobe(V, q, J, h, rep.w[m], nx * sgn[m], ny * sgn[m], nz * sgn[m], rep.kappa[m],
+                                    rep.norm[m], integ[m], out[0], out[1], out[2]);
+      pdf = m < KP ? fmaf(mw[m], v, pdf) : pdf;
+    }
     integral = sum;
   }
 }
 
-__global__ void __launch_bounds__(256) k_query(QueryField surf, QueryField vol, const HGRep* __restrict__ hg,
+template <bool VOLUMES>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VOLUMES ? 4 : 5))) k_query(QueryField surf, QueryField vol, const HGRep* __restrict__ hg,
                                                uint32_t n, const float* __restrict__ pos, const float* __restrict__ nrm,
                                                const float* __restrict__ gArr, const float* __restrict__ u2,
                                                const float* __restrict__ u1, const uint8_t* __restrict__ isVolume,
@@ -412,7 +473,7 @@ __global__ void __launch_bounds__(256) k_query(QueryField surf, QueryField vol, 
   const bool volume = isVolume ? isVolume[i] != 0 : false;
   float out[3], pdf, integral;
   uint32_t id;
-  query_quad(surf, vol, hg, volume, pos[3 * i], pos[3 * i + 1], pos[3 * i + 2], nrm[3 * i], nrm[3 * i + 1],
+  query_quad<VOLUMES>(surf, vol, hg, volume, pos[3 * i], pos[3 * i + 1], pos[3 * i + 2], nrm[3 * i], nrm[3 * i + 1],
              nrm[3 * i + 2], gArr ? gArr[i] : 0.f, u2[2 * i], u2[2 * i + 1], u1 ? u1[i] : -1.f, out, pdf, id, integral);
   if ((threadIdx.x & 3) != 0) return;
   dirOut[3 * i] = out[0];
@@ -426,7 +487,8 @@ __global__ void __launch_bounds__(256) k_query(QueryField surf, QueryField vol, 
 // Batch of pieces: the quad of query i of the batch finds its piece (pieces
 // ordered by begin) and works on query i - begin of it through the piece's
 // pointers.
-__global__ void __launch_bounds__(256) k_query_pieces(QueryField surf, QueryField vol, const HGRep* __restrict__ hg,
+template <bool VOLUMES>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VOLUMES ? 4 : 5))) k_query_pieces(QueryField surf, QueryField vol, const HGRep* __restrict__ hg,
                                                       const QueryPiece* __restrict__ pieces, uint32_t numPieces,
                                                       uint32_t n) {
   const uint32_t i = (uint32_t)(((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 2);
@@ -442,7 +504,7 @@ __global__ void __launch_bounds__(256) k_query_pieces(QueryField surf, QueryFiel
   const bool volume = P.vol ? P.vol[j] != 0 : false;
   float out[3], pdf, integral;
   uint32_t id;
-  query_quad(surf, vol, hg, volume, P.pos[3 * j], P.pos[3 * j + 1], P.pos[3 * j + 2], P.nrm[3 * j], P.nrm[3 * j + 1],
+  query_quad<VOLUMES>(surf, vol, hg, volume, P.pos[3 * j], P.pos[3 * j + 1], P.pos[3 * j + 2], P.nrm[3 * j], P.nrm[3 * j + 1],
              P.nrm[3 * j + 2], P.g ? P.g[j] : 0.f, P.u2[2 * j], P.u2[2 * j + 1], P.u1 ? P.u1[j] : -1.f, out, pdf, id,
              integral);
   if ((threadIdx.x & 3) != 0) return;
@@ -455,17 +517,17 @@ __global__ void __launch_bounds__(256) k_query_pieces(QueryField surf, QueryFiel
 }
 
 void launch_query_pieces(const QueryField& surf, const QueryField& vol, const HGRep* hg, const QueryPiece* pieces,
-                         uint32_t numPieces, uint32_t n, hipStream_t s) {
+                         uint32_t numPieces, uint32_t n, bool volumes, hipStream_t s) {
   if (n == 0 || numPieces == 0) return;
-  hipLaunchKernelGGL(k_query_pieces, dim3((n + 63) / 64), dim3(256), 0, s, surf, vol, hg, pieces, numPieces, n);
+  hipLaunchKernelGGL(volumes ? k_query_pieces<true> : k_query_pieces<false>, dim3((n + 63) / 64), dim3(256), 0, s, surf, vol, hg, pieces, numPieces, n);
 }
 
 void launch_query(const QueryField& surf, const QueryField& vol, const HGRep* hg, uint32_t n, const float* pos,
                   const float* nrm, const float* g, const float* u2, const float* u1, const uint8_t* isVolume,
                   float* dirOut, float* pdfOut, uint32_t* idOut, float* integralOut, hipStream_t s) {
   if (n == 0) return;
-  hipLaunchKernelGGL(k_query, dim3((n + 63) / 64), dim3(256), 0, s, surf, vol, hg, n, pos, nrm, g, u2, u1, isVolume,
-                     dirOut, pdfOut, idOut, integralOut);
+  hipLaunchKernelGGL(isVolume ? k_query<true> : k_query<false>, dim3((n + 63) / 64), dim3(256), 0, s, surf, vol, hg, n,
+                     pos, nrm, g, u2, u1, isVolume, dirOut, pdfOut, idOut, integralOut);
 }
 
 }  // namespace pglgpu

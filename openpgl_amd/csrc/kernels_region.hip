@@ -2003,6 +2003,7 @@ __device__ void region_job(Shared& sh, Team& tm, RegionState* __restrict__ state
     if (tid == 0) { S.valid = 0; S.splitFlag = 0; }
   }
   if (tid == 0) sh.S.prof[0] = (float)(wall_clock64() - tJob);
+  if (tid < 32) pack_query_comp(sh.S, tid);
   __syncthreads();
   if (tm.rank == 0) {
     uint32_t* dst = (uint32_t*)(states + r);

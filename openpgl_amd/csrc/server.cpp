@@ -270,6 +270,7 @@ void QueryServer::issue(Slot& s, std::vector<Piece>& batch, size_t N) {
   Arena a = carve(s.arena, slotQueries_);
   const auto tAdmit = std::chrono::steady_clock::now();
   size_t off = 0;
+  bool volumes = false;
   for (size_t k = 0; k < batch.size(); k++) {
     Piece& pc = batch[k];
     const QueryRequest& q = pc.req->q;
@@ -284,6 +285,7 @@ void QueryServer::issue(Slot& s, std::vector<Piece>& batch, size_t N) {
     QueryPiece& d = s.hostTable[k];
     d.begin = (uint32_t)off;
     d.n = (uint32_t)n;
+    volumes = volumes || q.isVolume != nullptr;
     if (pc.req->zeroCopy) {
       d.pos = q.pos + 3 * o;
       d.nrm = q.nrm + 3 * o;
@@ -319,7 +321,7 @@ void QueryServer::issue(Slot& s, std::vector<Piece>& batch, size_t N) {
   PGL_HIP_CHECK(hipMemcpyAsync(s.devTable, s.hostTable, batch.size() * sizeof(QueryPiece), hipMemcpyHostToDevice,
                                s.stream));
   launch_query_pieces(surf_[s.snap].view, vol_[s.snap].view, gf_->dHG.as<HGRep>(), s.devTable, (uint32_t)batch.size(),
-                      (uint32_t)N, s.stream);
+                      (uint32_t)N, volumes, s.stream);
   PGL_HIP_CHECK(hipGetLastError());
   off = 0;
   for (auto& pc : batch) {
