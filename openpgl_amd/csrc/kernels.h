@@ -165,6 +165,22 @@ void launch_query(const QueryField& surf, const QueryField& vol, const HGRep* hg
 struct PathSampleOptions;
 struct PathSample;
 size_t path_scan_temp_bytes(uint32_t numSegments);
+// The same records in one pass over the vertices, written straight to outputs
+// that hold every vertex; paths longer than kFusedPathLength, or long runs of
+// vertices that no path holds, are left to the launches above: totals (memory
+// that the device writes and the host reads after a synchronisation): [0], [1],
+// [2] as above, [3] 1 if nothing was written.  control is zeroed once before
+// its first use, epoch another number > 0 for every launch.
+constexpr uint32_t kFusedPathLength = 64;
+constexpr uint32_t kFusedPathVertices = 1u << 26;  // at most this many
+struct FusedPathControl {
+  uint32_t ticket;        // next tile
+  uint32_t bad, general;  // epoch of the launch that met such paths
+};
+void launch_path_fused(const PathVertex* segs, uint32_t numSegments, const uint32_t* offsets, uint32_t numPaths,
+                       const PathSampleOptions& o, PathSample* surfOut, PathSample* volOut, uint32_t* tileFirst,
+                       unsigned long long* tileWord, FusedPathControl* control, uint32_t epoch, uint32_t numCUs,
+                       unsigned long long* totals, hipStream_t s);
 size_t path_tile_words(uint32_t numSegments);  // entries of tileFirst
 void launch_path_records(const PathVertex* segs, uint32_t numSegments, const uint32_t* offsets, uint32_t numPaths,
                          const PathSampleOptions& o, PathSample* records, unsigned long long* flags, uint32_t* pathOf,

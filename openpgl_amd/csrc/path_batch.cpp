@@ -11,6 +11,7 @@ static_assert(sizeof(PathSample) == kSampleRecordBytes, "PathSample is the 40-by
 
 PathSampleBatch::PathSampleBatch() {
   PGL_HIP_CHECK(hipStreamCreate(&stream_));
+  hTotals_.coherent = true;
 }
 
 PathSampleBatch::~PathSampleBatch() {
@@ -24,7 +25,7 @@ void PathSampleBatch::count(const PathVertex* segs, uint32_t numSegments, const 
   offsets_ = offsets;
   numSegments_ = numPaths ? numSegments : 0;
   totals_.ensure(24);
-  hTotals_.ensure(24);
+  hTotals_.ensure(32);
   const size_t V = std::max<size_t>(numSegments_, 1);
   records_.ensure(V * sizeof(PathSample));
   flags_.ensure(V * 8);
@@ -51,9 +52,42 @@ void PathSampleBatch::scatter(PathSample* surfOut, PathSample* volOut) {
   PGL_HIP_CHECK(hipStreamSynchronize(stream_));
 }
 
+bool PathSampleBatch::fused(const PathVertex* segs, uint32_t numSegments, const uint32_t* offsets, uint32_t numPaths,
+                            const PathSampleOptions& o, PathSample* surfOut, PathSample* volOut, size_t& numSurf,
+                            size_t& numVol) {
+  numSurf = numVol = 0;
+  if (numPaths == 0 || numSegments == 0) return true;
+  const size_t tiles = path_tile_words(numSegments);
+  tiles_.ensure(tiles * 4);
+  tileWords_.ensure(tiles * 16);
+  hTotals_.ensure(32);
+  if (!control_.p) {
+    int dev = 0, cus = 0;
+    PGL_HIP_CHECK(hipGetDevice(&dev));
+    PGL_HIP_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    numCUs_ = (uint32_t)cus;
+    control_.ensure(sizeof(FusedPathControl));
+    PGL_HIP_CHECK(hipMemsetAsync(control_.p, 0, sizeof(FusedPathControl), stream_));
+  }
+  if (++epoch_ == 0) epoch_ = 1;
+  launch_path_fused(segs, numSegments, offsets, numPaths, o, surfOut, volOut, tiles_.as<uint32_t>(),
+                    tileWords_.as<unsigned long long>(), control_.as<FusedPathControl>(), epoch_, numCUs_,
+                    (unsigned long long*)hTotals_.dev, stream_);
+  PGL_HIP_CHECK(hipStreamSynchronize(stream_));
+  const unsigned long long* t = hTotals_.as<unsigned long long>();
+  if (t[2]) throw std::runtime_error("openpgl_amd: path offsets must be non-decreasing and within the segments");
+  if (t[3]) return false;
+  numSurf = (size_t)t[0];
+  numVol = (size_t)t[1];
+  return true;
+}
+
 void PathSampleBatch::prepare(const PathVertex* segs, uint32_t numSegments, const uint32_t* offsets,
                               uint32_t numPaths, const PathSampleOptions& o, PathSample* surfOut, size_t surfCap,
                               PathSample* volOut, size_t volCap, size_t& numSurf, size_t& numVol) {
+  if (surfCap >= numSegments && volCap >= numSegments && numSegments <= kFusedPathVertices &&
+      fused(segs, numSegments, offsets, numPaths, o, surfOut, volOut, numSurf, numVol))
+    return;
   count(segs, numSegments, offsets, numPaths, o, numSurf, numVol);
   if (numSurf > surfCap || numVol > volCap)
     throw std::runtime_error("openpgl_amd: path samples exceed the output capacity (" + std::to_string(numSurf) +
@@ -66,6 +100,17 @@ void PathSampleBatch::prepareOwned(const PathVertex* segs, uint32_t numSegments,
                                    uint32_t numPaths, const PathSampleOptions& o, const PathSample*& surf,
                                    size_t& numSurf, const PathSample*& vol, size_t& numVol) {
   const int b = next_;
+  if (numSegments <= kFusedPathVertices) {
+    acquireOwned(b, numSegments, numSegments);
+    if (fused(segs, numSegments, offsets, numPaths, o, out_[b][0].as<PathSample>(), out_[b][1].as<PathSample>(),
+              numSurf, numVol)) {
+      next_ = 1 - next_;
+      surf = out_[b][0].as<PathSample>();
+      vol = out_[b][1].as<PathSample>();
+      lastBuffer_ = b;
+      return;
+    }
+  }
   count(segs, numSegments, offsets, numPaths, o, numSurf, numVol);
   next_ = 1 - next_;
   acquireOwned(b, numSurf, numVol);
@@ -94,7 +139,7 @@ void PathSampleBatch::routeOwned(const PathSample* recs, uint32_t n, const PathS
   const int b = next_;
   next_ = 1 - next_;
   totals_.ensure(24);
-  hTotals_.ensure(24);
+  hTotals_.ensure(32);
   const size_t V = std::max<size_t>(n, 1);
   flags_.ensure(V * 8);
   incl_.ensure(V * 8);

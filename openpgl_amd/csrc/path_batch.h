@@ -20,7 +20,8 @@ class PathSampleBatch {
   // a range outside [0, numSegments] is an error),
   // then writes them to surfOut / volOut (device, capacities in records).
   // Throws if a capacity is too small (nothing is written then).  Blocks
-  // until the records are written.
+  // until the records are written.  Outputs with room for every vertex are
+  // written in one pass, without counting first.
   void prepare(const PathVertex* segs, uint32_t numSegments, const uint32_t* offsets, uint32_t numPaths,
                const PathSampleOptions& o, PathSample* surfOut, size_t surfCap, PathSample* volOut, size_t volCap,
                size_t& numSurf, size_t& numVol);
@@ -46,11 +47,17 @@ class PathSampleBatch {
   void count(const PathVertex* segs, uint32_t numSegments, const uint32_t* offsets, uint32_t numPaths,
              const PathSampleOptions& o, size_t& numSurf, size_t& numVol);
   void scatter(PathSample* surfOut, PathSample* volOut);
+  // one pass into outputs that hold every vertex; false (and nothing written)
+  // where the paths need the counting launches
+  bool fused(const PathVertex* segs, uint32_t numSegments, const uint32_t* offsets, uint32_t numPaths,
+             const PathSampleOptions& o, PathSample* surfOut, PathSample* volOut, size_t& numSurf, size_t& numVol);
   // output buffer b for ns / nv records, once its previous consumers are done
   void acquireOwned(int b, size_t numSurf, size_t numVol);
 
   hipStream_t stream_ = nullptr;
   DevBuf records_, flags_, pathOf_, tiles_, incl_, scanTemp_, totals_;
+  DevBuf tileWords_, control_;  // of fused()
+  uint32_t epoch_ = 0, numCUs_ = 0;
   const uint32_t* offsets_ = nullptr;  // of the last count()
   uint32_t numSegments_ = 0;
   PinnedBuf hTotals_;

@@ -10,6 +10,7 @@
 // compiles it with contraction off.
 #pragma once
 #include <math.h>
+#include <string.h>
 
 #include "common.h"
 
@@ -32,51 +33,95 @@ PGL_HD inline float path_fdot(float ax, float ay, float az, float bx, float by, 
   return fmaf(ax, bx, fmaf(ay, by, az * bz));
 }
 
-// One step of the backward walk at vertex c (next vertex nx): the sample
-// distance of c and the length carried on to the previous vertex.
-PGL_HD inline float path_step_distance(const PathVertex& c, const PathVertex& nx, float maxDistance,
-                                       float& lastDistance) {
-  // distance to the next vertex plus the length carried through specular chains
+// What vertex c adds to a backward walk (next vertex nx): the distance between
+// the two, and the factor of the length carried on to the previous vertex
+// (kPathEnds where a rough vertex ends the specular chain).
+constexpr float kPathEnds = -1.0f;
+PGL_HD inline float path_edge(const PathVertex& c, const PathVertex& nx, float& factor) {
   const float ex = nx.px - c.px, ey = nx.py - c.py, ez = nx.pz - c.pz;
-  const float currentDistance = sqrtf(path_fdot(ex, ey, ez, ex, ey, ez));
-  const float distance = fminf(currentDistance + lastDistance, 2.0f * maxDistance);
-  if (!c.isDelta && c.roughness >= 0.3f) {
-    lastDistance = 0.0f;
-  } else {
-    lastDistance = distance;
+  factor = kPathEnds;
+  if (c.isDelta || !(c.roughness >= 0.3f)) {
+    factor = 1.0f;
     if (c.eta != 1.0f) {
       const float cosThetaI = path_fdot(c.nx, c.ny, c.nz, c.dox, c.doy, c.doz);
       const float cosThetaO = path_fdot(c.nx, c.ny, c.nz, c.dix, c.diy, c.diz);
-      lastDistance *= fabsf(cosThetaI / (cosThetaO * c.eta));
+      factor = fabsf(cosThetaI / (cosThetaO * c.eta));
     }
   }
+  return sqrtf(path_fdot(ex, ey, ez, ex, ey, ez));
+}
+
+// One step of the walk: the sample distance of the vertex, and the length
+// carried on (the distance to the next vertex plus that of specular chains).
+PGL_HD inline float path_carry(float edge, float factor, float maxDistance, float& lastDistance) {
+  const float distance = fminf(edge + lastDistance, 2.0f * maxDistance);
+  lastDistance = factor == kPathEnds ? 0.0f : distance * factor;
   return distance;
 }
 
+// The sample distance of c (next vertex nx) and the length carried on.
+PGL_HD inline float path_step_distance(const PathVertex& c, const PathVertex& nx, float maxDistance,
+                                       float& lastDistance) {
+  float factor;
+  const float edge = path_edge(c, nx, factor);
+  return path_carry(edge, factor, maxDistance, lastDistance);
+}
+
+// delta and near-specular vertices yield no sample
+PGL_HD inline bool path_vertex_records(const PathVertex& c) { return !c.isDelta && c.roughness > 0.01f; }
+
+// What a vertex contributes to the walks of the vertices before it.
+struct PathStep {
+  float scattering[3], transmittance[3], direct[3], miWeight, scattered[3], survival, reciprocal;
+};
+PGL_HD inline PathStep path_step(const PathVertex& v) {
+  PathStep s;
+  for (int k = 0; k < 3; k++) {
+    s.scattering[k] = v.scatteringWeight[k];
+    s.transmittance[k] = v.transmittanceWeight[k];
+    s.direct[k] = v.directContribution[k];
+    s.scattered[k] = v.scatteredContribution[k];
+  }
+  s.miWeight = v.miWeight;
+  s.survival = v.russianRouletteProbability;
+  memcpy(&s.reciprocal, &v.pad2, 4);  // of use to those that kept one there
+  return s;
+}
+
+struct DivideBySurvival {
+  PGL_HD void operator()(const PathStep& v, float t[3]) const {
+    for (int k = 0; k < 3; k++) t[k] /= v.survival;
+  }
+};
+
 // The sample of vertex i (sample distance given), or false when vertex i
 // yields none: delta or near-specular vertex, no radiance brought back, or a
-// non-positive distance.
+// non-positive distance.  divide(v, t): t over v's survival probability.
+template <class Divide = DivideBySurvival>
 PGL_HD inline bool path_vertex_record(const PathVertex* seg, int n, int i, float distance, const PathSampleOptions& o,
-                                      PathSample& s) {
+                                      PathSample& s, Divide&& divide = Divide()) {
   const float minPdf = 0.1f;
   const float maxThroughput = 10.0f;
   const PathVertex& c = seg[i];
-  if (c.isDelta || !(c.roughness > 0.01f)) return false;
+  if (!path_vertex_records(c)) return false;
   const float pdf = minPdf < c.pdfDirectionIn ? c.pdfDirectionIn : minPdf;
   // incident radiance carried back from the rest of the path
   float t[3] = {1.0f, 1.0f, 1.0f};
   float contrib[3] = {0.0f, 0.0f, 0.0f};
   float previousRR = 1.0f;
+  float passed[3] = {c.transmittanceWeight[0], c.transmittanceWeight[1], c.transmittanceWeight[2]};
+  PathStep ahead = path_step(seg[i + 1 < n ? i + 1 : i]);  // read one step ahead of its use
+#pragma unroll 2
   for (int j = i + 1; j < n; ++j) {
-    const PathVertex& prev = seg[j - 1];
-    const PathVertex& v = seg[j];
+    const PathStep v = ahead;
+    ahead = path_step(seg[j + 1 < n ? j + 1 : j]);
     float ct[3];
     for (int k = 0; k < 3; k++) {
-      t[k] = t[k] * prev.transmittanceWeight[k];
+      t[k] = t[k] * passed[k];
       ct[k] = t[k] < maxThroughput ? t[k] : maxThroughput;
-      contrib[k] += ct[k] * v.scatteredContribution[k];
+      contrib[k] += ct[k] * v.scattered[k];
     }
-    float direct[3] = {v.directContribution[0], v.directContribution[1], v.directContribution[2]};
+    float direct[3] = {v.direct[0], v.direct[1], v.direct[2]};
     if (!o.rrAffectsDirectContribution)
       for (int k = 0; k < 3; k++) direct[k] *= previousRR;
     if (j == i + 1 && !o.useNEEMiWeights) {
@@ -85,14 +130,14 @@ PGL_HD inline bool path_vertex_record(const PathVertex* seg, int n, int i, float
     } else if (j > i + 1 || o.guideDirectLight) {
       for (int k = 0; k < 3; k++) contrib[k] += (ct[k] * v.miWeight) * direct[k];
     }
-    for (int k = 0; k < 3; k++) t[k] = t[k] * v.scatteringWeight[k];
-    const float rr = v.russianRouletteProbability;
-    if (rr > 0.f) {
-      for (int k = 0; k < 3; k++) t[k] /= rr;
+    for (int k = 0; k < 3; k++) t[k] = t[k] * v.scattering[k];
+    if (v.survival > 0.f) {
+      divide(v, t);
     } else {
       t[0] = t[1] = t[2] = 0.0f;
     }
-    previousRR = rr;
+    previousRR = v.survival;
+    for (int k = 0; k < 3; k++) passed[k] = v.transmittance[k];
   }
   if (!(contrib[0] > 0.0f || contrib[1] > 0.0f || contrib[2] > 0.0f)) return false;
   if (!(distance > 0.0f)) return false;

@@ -120,3 +120,50 @@ def test_field_update_from_path_segments():
             ra, rb = a.region(i, kind), b.region(i, kind)
             for key in ("K", "weights", "kappas", "meanDirections", "ssMean", "numSamplesThisUpdate"):
                 assert np.array_equal(np.asarray(ra[key]), np.asarray(rb[key])), (kind, i, key)
+
+
+_SHAPES = {
+    "one vertex": ([1], 0, 0),
+    "two vertices": ([2], 0, 0),
+    "last path begins at a tile's last vertex": ([3] * 85 + [64] + [5] * 3, 0, 0),
+    "paths end with the tiles": ([64] * 8, 0, 0),
+    "longest one-pass path, then one more": ([64, 65, 7], 0, 0),
+    "read-ahead ends inside a path": ([16] * 15 + [15, 17, 2], 0, 0),
+    "vertices of no path": ([12] * 60, 300, 300),
+    "long runs of them": ([12] * 60, 70 * 256, 70 * 256),
+    "tiles of two passes of the sums": ([8] * (520 * 32), 0, 0),
+}
+
+
+@pytest.mark.parametrize("shape", list(_SHAPES))
+def test_one_pass_equals_counting(shape):
+    """Outputs with room for every vertex (one pass) and outputs of just the
+    records' size (counting first) hold the oracle's records, bit for bit; with
+    survival probabilities and throughputs from denormal to huge, where a
+    quotient is not formed from a kept reciprocal."""
+    import openpgl_amd as pgl
+    from openpgl_amd.hip_runtime import DeviceArray
+    lengths, lead, trail = _SHAPES[shape]
+    n = lead + sum(lengths) + trail
+    rng = np.random.Generator(np.random.PCG64([n, 99]))
+    seg, _ = random_paths(n // 5 + 8, seed=31, max_len=12)
+    seg = seg[:n].copy()
+    assert len(seg) == n
+    seg["roughness"] = np.maximum(seg["roughness"], 0.02)
+    rr = "russianRouletteProbability"
+    seg[rr] = rng.choice(np.array([1.0, 0.7, 0.95, 3e-39, 1e-30, 2e-18, 9e-19, 1e6, 2e6, 1e30], np.float32), n,
+                         p=[.3, .3, .2] + [.2 / 7] * 7)
+    seg["scatteringWeight"] *= rng.choice(np.array([1.0, 0.0, 1e-20, 1e-38, 1e25], np.float32), (n, 1),
+                                          p=[.8, .05, .05, .05, .05])
+    off = (lead + np.concatenate([[0], np.cumsum(lengths)])).astype(np.uint32)
+    print(shape, "paths", len(lengths), "vertices", n, flush=True)
+    batch = pgl.PathSegmentBatch()
+    ws, wv = oracle_path_samples(seg, off)
+    s, v = _device_samples(batch, seg, off)
+    assert s.tobytes() == ws.tobytes() and v.tobytes() == wv.tobytes()
+    dseg, doff = DeviceArray.from_numpy(seg), DeviceArray.from_numpy(off)
+    ds, dv = DeviceArray(40 * max(1, len(ws))), DeviceArray(40 * max(1, len(wv)))
+    r = batch.prepare_device(dseg.value, n, doff.value, len(lengths), ds.value, len(ws), dv.value, len(wv))
+    assert r == (len(ws), len(wv))
+    assert ds.to_numpy(SAMPLE_DTYPE, (len(ws),)).tobytes() == ws.tobytes()
+    assert dv.to_numpy(SAMPLE_DTYPE, (len(wv),)).tobytes() == wv.tobytes()
