@@ -1,0 +1,84 @@
+"""The region kernel at the edges of its loops: sample counts around a wave, a
+workgroup and a chunk, component counts of every number of groups, directions
+that leave the range the bounded exponent assumes, and launches on either side
+of the default grid's rule.
+
+Against the oracle (as the batched launch, tests/parity_checks.py) and bit for
+bit between schedules: how a region's samples are shared out changes no result.
+"""
+import numpy as np
+import pytest
+
+from field_compare import unit_dirs
+from parity_checks import assert_mixture_parity
+from test_gpu_batch import _oracle_regions, _state
+from openpgl_amd.synth import batched_regions
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [64, 65, 127, 128, 129, 255, 256, 257, 511, 512, 513, 1023, 1024, 1025, 2047, 2048, 2049, 4097]
+
+
+def _regions(counts, ks, seed):
+    """region r: the first counts[r] of its samples, ks[r] initial components"""
+    n = int(max(counts))
+    full, have, _, _ = batched_regions(len(counts), seed=seed, nmin=n, nmax=n + 0.5)
+    assert (have == n).all()
+    recs = np.concatenate([full[r * n:r * n + c] for r, c in enumerate(counts)])
+    stats = np.zeros((len(counts), 7), np.float32)
+    at = 0
+    for r, c in enumerate(counts):
+        p = recs["pos"][at:at + c].astype(np.float64)
+        stats[r, 0:3] = p.mean(axis=0)
+        stats[r, 3:6] = ((p - p.mean(axis=0)) ** 2).sum(axis=0)
+        stats[r, 6] = c
+        at += c
+    return recs, np.asarray(counts, np.uint32), stats, np.asarray(ks, np.uint32)
+
+
+def _run(recs, counts, stats, init_k, **schedule):
+    import openpgl_amd as pgl
+    from openpgl_amd.hip_runtime import DeviceArray
+    batch = pgl.RegionBatch(pgl.Device(), max_samples_per_leaf=32000)
+    if schedule:
+        batch.set_schedule(**schedule)
+    print("regions", len(counts), "samples", len(recs), "schedule", schedule, flush=True)
+    batch.samples = DeviceArray.from_numpy(recs)  # kept with the batch, which reads it after the call
+    batch.step_device(batch.samples.value, counts, stats, init_k)
+    return batch
+
+
+@pytest.mark.parametrize("k", [8, 9, 12, 16, 20, 24, 28, 31, 32])
+def test_sample_counts_and_groups(k):
+    recs, counts, stats, init_k = _regions(EDGES, [k] * len(EDGES), seed=40 + k)
+    batch = _run(recs, counts, stats, init_k)
+    records = [batch.region(r) for r in range(len(counts))]
+    o32 = _oracle_regions(recs, counts, stats, init_k, [(recs, stats)], 0)
+    o64 = _oracle_regions(recs, counts, stats, init_k, [(recs, stats)], 1)
+    assert_mixture_parity(records, [o.record() for o in o32], [o.record() for o in o64], unit_dirs(512), "K %d" % k)
+    assert _state(batch) == _state(_run(recs, counts, stats, init_k, per_region_launches=1))
+    assert _state(batch) == _state(_run(recs, counts, stats, init_k, per_region_launches=0, balance=8.0, max_team=64))
+
+
+@pytest.mark.parametrize("scale", [1.5, 30.0])
+def test_directions_out_of_range(scale):
+    """a region with directions longer than one takes the loops that bound no
+    exponent: the same bits alone and in teams, its neighbours' bits unchanged"""
+    counts, ks = [300, 5000, 300], [8, 20, 32]
+    recs, c, stats, init_k = _regions(counts, ks, seed=7)
+    plain = _state(_run(recs, c, stats, init_k))
+    recs = recs.copy()
+    recs["dir"][300 + 17:300 + 5000:100] *= np.float32(scale)
+    ref = _state(_run(recs, c, stats, init_k, per_region_launches=1))
+    assert ref[0] == plain[0] and ref[2] == plain[2]
+    assert ref == _state(_run(recs, c, stats, init_k))
+    assert ref == _state(_run(recs, c, stats, init_k, per_region_launches=0, balance=8.0, max_team=64))
+
+
+@pytest.mark.parametrize("counts", [[96 + r % 5 for r in range(511)], [96 + r % 5 for r in range(700)],
+                                    [100000 + 777 * r for r in range(36)]])
+def test_default_grid_rule(counts):
+    """fewer and more regions than the default grid has workgroups, and more
+    chunks than it takes at once, against a small fixed grid"""
+    recs, c, stats, init_k = _regions(counts, [(8, 16, 32)[r % 3] for r in range(len(counts))], seed=3)
+    assert _state(_run(recs, c, stats, init_k)) == _state(_run(recs, c, stats, init_k, grid=96))
