@@ -113,8 +113,10 @@ __device__ __forceinline__ float qlane(float v) {
 // Correctly rounded n / d by the steps of the compiler's division (one
 // refinement of the reciprocal, two of the quotient), the reciprocal formed
 // once per d, without the scaling that only operands near the ends of the
-// exponent range need: the same quotient while d and n / d lie within
-// 2^-100 .. 2^100 (or n is 0).
+// exponent range need: the same quotient while d, n and n / d lie within
+// 2^-100 .. 2^100 (or n is 0).  A smaller n, whose remainders are rounded to
+// denormals, may end a unit in the last place off: a coordinate under 2^-50 of
+// its vector's length, or a component's share under 2^-33 of the integral.
 struct Recip {
   float d, r;
 };
@@ -162,17 +164,20 @@ __device__ __forceinline__ void lane_shift(const Mixture& V, int k, bool par, fl
   mz = a.z;
   if (par) {  // shift_comp
     const float d = a.w;
+    const bool shift = d > 0.f && isfinite(d);
     const float px = fmaf(mx, d, sx), py = fmaf(my, d, sy), pz = fmaf(mz, d, sz);
-    const float l = sqrt_in_range(qdot(px, py, pz, px, py, pz));
+    const float l2 = qdot(px, py, pz, px, py, pz);
+    const float l = sqrt_in_range(l2);
     const Recip rl = recip_of(l);
     float qx = div_by(px, rl), qy = div_by(py, rl), qz = div_by(pz, rl);
-    // a distance whose square leaves the exponent range (a component may carry any)
-    if (__ballot(!(l > 1e-15f && l < 1e18f)) != 0) {
-      qx = px / l;
-      qy = py / l;
-      qz = pz / l;
+    // a length out of the root's or the quotients' range (a component may carry
+    // any distance): the scaled forms, which give the other lanes the same bits
+    if (__ballot(shift && !(l > 1e-13f && l < 1e18f)) != 0) {
+      const float ls = sqrtf(l2);
+      qx = px / ls;
+      qy = py / ls;
+      qz = pz / ls;
     }
-    const bool shift = d > 0.f && isfinite(d);
     mx = shift ? qx : mx;
     my = shift ? qy : my;
     mz = shift ? qz : mz;
