@@ -162,6 +162,7 @@ void launch_query(const QueryField& surf, const QueryField& vol, const HGRep* hg
 // path segments -> training samples (kernels_path.hip).  Per vertex: its
 // record, a flag packed as surface | volume << 32 and its path; totals:
 // [0] surface records, [1] volume records, [2] 1 if a path range was malformed
+// (checked: known not to be, [2] is left as it is)
 struct PathSampleOptions;
 struct PathSample;
 size_t path_scan_temp_bytes(uint32_t numSegments);
@@ -185,7 +186,7 @@ size_t path_tile_words(uint32_t numSegments);  // entries of tileFirst
 void launch_path_records(const PathVertex* segs, uint32_t numSegments, const uint32_t* offsets, uint32_t numPaths,
                          const PathSampleOptions& o, PathSample* records, unsigned long long* flags, uint32_t* pathOf,
                          uint32_t* tileFirst, unsigned long long* incl, void* scanTemp, size_t scanBytes,
-                         unsigned long long* totals, hipStream_t s);
+                         bool checked, unsigned long long* totals, hipStream_t s);
 void launch_path_scatter(const PathSample* records, const unsigned long long* flags, const uint32_t* pathOf,
                          const unsigned long long* incl, const uint32_t* offsets, uint32_t numSegments,
                          PathSample* surfOut, PathSample* volOut, hipStream_t s);

@@ -657,11 +657,12 @@ size_t path_tile_words(uint32_t numSegments) { return (numSegments + kPathThread
 void launch_path_records(const PathVertex* segs, uint32_t numSegments, const uint32_t* offsets, uint32_t numPaths,
                          const PathSampleOptions& o, PathSample* records, unsigned long long* flags, uint32_t* pathOf,
                          uint32_t* tileFirst, unsigned long long* incl, void* scanTemp, size_t scanBytes,
-                         unsigned long long* totals, hipStream_t s) {
-  hipLaunchKernelGGL(k_path_clear, dim3(1), dim3(64), 0, s, totals);
+                         bool checked, unsigned long long* totals, hipStream_t s) {
+  if (!checked) hipLaunchKernelGGL(k_path_clear, dim3(1), dim3(64), 0, s, totals);
   if (numPaths == 0 || numSegments == 0) return;
-  hipLaunchKernelGGL(k_path_check, dim3((numPaths + kPathThreads - 1) / kPathThreads), dim3(kPathThreads), 0, s,
-                     offsets, numPaths, numSegments, totals);
+  if (!checked)
+    hipLaunchKernelGGL(k_path_check, dim3((numPaths + kPathThreads - 1) / kPathThreads), dim3(kPathThreads), 0, s,
+                       offsets, numPaths, numSegments, totals);
   const uint32_t numTiles = (numSegments + kPathThreads - 1) / kPathThreads;
   hipLaunchKernelGGL(k_path_tiles, dim3(numTiles / kPathThreads + 1), dim3(kPathThreads), 0, s, offsets, numPaths,
                      numSegments, numTiles, tileFirst);
@@ -761,7 +762,7 @@ void path_prepare_noalloc(const PathVertex* segs, uint32_t numSegments, const ui
   const size_t scanBytes = path_scan_temp_bytes(n > 0 ? n : 1u);
   if (scanBytes > kNaScanBytes) throw std::runtime_error("openpgl_amd: path scan storage exceeds the static scratch");
   launch_path_records(segs, n, offsets, numPaths, o, records, flags, pathOf, tiles, incl, base + kNaScan, scanBytes,
-                      totals, s);
+                      false, totals, s);
   unsigned long long t[3] = {0ull, 0ull, 0ull};
   PGL_KERNEL_CHECK(hipMemcpyAsync(t, totals, sizeof(t), hipMemcpyDeviceToHost, s));
   PGL_KERNEL_CHECK(hipStreamSynchronize(s));

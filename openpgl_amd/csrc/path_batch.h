@@ -44,12 +44,16 @@ class PathSampleBatch {
   hipStream_t stream() const { return stream_; }
 
  private:
+  // the counting launches into scratch (checked: the offsets are known to be
+  // well formed), and the records from there to their outputs; neither waits
   void count(const PathVertex* segs, uint32_t numSegments, const uint32_t* offsets, uint32_t numPaths,
-             const PathSampleOptions& o, size_t& numSurf, size_t& numVol);
+             const PathSampleOptions& o, bool checked);
   void scatter(PathSample* surfOut, PathSample* volOut);
-  // one pass into outputs that hold every vertex; false (and nothing written)
-  // where the paths need the counting launches
-  bool fused(const PathVertex* segs, uint32_t numSegments, const uint32_t* offsets, uint32_t numPaths,
+  // waits and reads the totals (throws for malformed offsets); false if the one pass left the paths
+  bool totals(size_t& numSurf, size_t& numVol);
+  // into outputs that hold every vertex: one pass, or the counting launches
+  // where the paths need them; blocks
+  void fused(const PathVertex* segs, uint32_t numSegments, const uint32_t* offsets, uint32_t numPaths,
              const PathSampleOptions& o, PathSample* surfOut, PathSample* volOut, size_t& numSurf, size_t& numVol);
   // output buffer b for ns / nv records, once its previous consumers are done
   void acquireOwned(int b, size_t numSurf, size_t numVol);

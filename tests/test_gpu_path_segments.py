@@ -122,6 +122,31 @@ def test_field_update_from_path_segments():
                 assert np.array_equal(np.asarray(ra[key]), np.asarray(rb[key])), (kind, i, key)
 
 
+@pytest.mark.parametrize("lengths", [[64, 65, 64], [8, 300, 8]])
+def test_field_update_with_and_without_long_paths(lengths):
+    """Frames whose longest path has lengths[frame] vertices, so that the one
+    pass and the counting launches alternate on one field: the states of a field
+    trained from the oracle's records of the same paths."""
+    import openpgl_amd as pgl
+    from openpgl_amd.hip_runtime import DeviceArray
+    dev = pgl.Device()
+    a = pgl.Field(dev, max_samples_per_leaf=2000)
+    b = pgl.Field(dev, max_samples_per_leaf=2000)
+    for frame, longest in enumerate(lengths):
+        seg, off = random_paths(20000, seed=200 + frame, max_len=8)
+        at = int(off[7000])  # one path of `longest` vertices, empty paths behind it
+        off = np.where((off > at) & (off < at + longest), at + longest, off).astype(np.uint32)
+        print("frame", frame, "vertices", len(seg), "longest", int(np.diff(off).max()), flush=True)
+        assert longest <= np.diff(off).max() < longest + 8
+        dseg, doff = DeviceArray.from_numpy(seg), DeviceArray.from_numpy(off)
+        a.update_from_path_segments_device(dseg.value, len(seg), doff.value, len(off) - 1)
+        ws, wv = oracle_path_samples(seg, off)
+        b.update(pgl.SampleStorage(np.concatenate([ws, wv])))
+        assert a.iteration() == b.iteration() == frame + 1
+    assert a.num_regions(0) > 4 and a.num_regions(1) > 1
+    assert a.compare(b)
+
+
 _SHAPES = {
     "one vertex": ([1], 0, 0),
     "two vertices": ([2], 0, 0),
