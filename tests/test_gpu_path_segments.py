@@ -157,6 +157,9 @@ _SHAPES = {
     "vertices of no path": ([12] * 60, 300, 300),
     "long runs of them": ([12] * 60, 70 * 256, 70 * 256),
     "tiles of two passes of the sums": ([8] * (520 * 32), 0, 0),
+    "most paths of a tile taken one by one": ([4] * 32 + [0] * 1984 + [4] * 112, 0, 0),
+    "one more": ([4] * 32 + [0] * 1985 + [4] * 112, 0, 0),
+    "a tile of empty paths, then a path into the next": ([0] * 3000 + [7] * 30 + [0] * 3000 + [64, 7], 11, 5),
 }
 
 
@@ -192,3 +195,30 @@ def test_one_pass_equals_counting(shape):
     assert r == (len(ws), len(wv))
     assert ds.to_numpy(SAMPLE_DTYPE, (len(ws),)).tobytes() == ws.tobytes()
     assert dv.to_numpy(SAMPLE_DTYPE, (len(wv),)).tobytes() == wv.tobytes()
+
+
+def test_runs_of_empty_paths_cost_little():
+    """Half a million empty paths between the paths of a small frame (rays that
+    left the scene): the call stays in the time of the frame without them."""
+    import time
+    import openpgl_amd as pgl
+    from openpgl_amd.hip_runtime import DeviceArray
+    seg, off = random_paths(2000, seed=5, max_len=12)
+    mid = len(off) // 2
+    batch = pgl.PathSegmentBatch()
+    best, counts = [], []
+    for empty in (0, 500000):
+        o = np.concatenate([off[:mid], np.full(empty, off[mid], np.uint32), off[mid:]]).astype(np.uint32)
+        print("empty paths", empty, flush=True)
+        n = len(seg)
+        dseg, doff = DeviceArray.from_numpy(seg), DeviceArray.from_numpy(o)
+        ds, dv = DeviceArray(40 * n), DeviceArray(40 * n)
+        times = []
+        for _ in range(20):
+            t = time.perf_counter()
+            r = batch.prepare_device(dseg.value, n, doff.value, len(o) - 1, ds.value, n, dv.value, n)
+            times.append(time.perf_counter() - t)
+        best.append(min(times))
+        counts.append((r, ds.to_numpy(SAMPLE_DTYPE, (r[0],)).tobytes()))
+    assert counts[0] == counts[1]
+    assert best[1] < 4 * best[0], best
