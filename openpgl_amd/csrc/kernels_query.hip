@@ -164,20 +164,19 @@ __device__ __forceinline__ void lane_shift(const Mixture& V, int k, bool par, fl
   mz = a.z;
   if (par) {  // shift_comp
     const float d = a.w;
-    const bool shift = d > 0.f && isfinite(d);
     const float px = fmaf(mx, d, sx), py = fmaf(my, d, sy), pz = fmaf(mz, d, sz);
-    const float l2 = qdot(px, py, pz, px, py, pz);
-    const float l = sqrt_in_range(l2);
+    const float l = sqrt_in_range(qdot(px, py, pz, px, py, pz));
     const Recip rl = recip_of(l);
     float qx = div_by(px, rl), qy = div_by(py, rl), qz = div_by(pz, rl);
     // a length out of the root's or the quotients' range (a component may carry
     // any distance): the scaled forms, which give the other lanes the same bits
-    if (__ballot(shift && !(l > 1e-13f && l < 1e18f)) != 0) {
-      const float ls = sqrtf(l2);
+    if (__ballot(!(l > 1e-13f && l < 1e18f)) != 0) {
+      const float ls = sqrtf(qdot(px, py, pz, px, py, pz));
       qx = px / ls;
       qy = py / ls;
       qz = pz / ls;
     }
+    const bool shift = d > 0.f && isfinite(d);  // (formed before the divisions: 277 instead of 261 us, above)
     mx = shift ? qx : mx;
     my = shift ? qy : my;
     mz = shift ? qz : mz;
