@@ -366,8 +366,9 @@ size_t pglFieldGetUpdateHistory(PGLField field, int kind, double* out, size_t ma
  *                      device; 0: one persistent launch
  *   grid               workgroups of the persistent launch (0: two per CU,
  *                      which leaves room for other streams' kernels, and
- *                      most of the three that fit for launches of more
- *                      regions or 1024-sample chunks than those can share;
+ *                      the three that fit less the larger of 64 and
+ *                      maxTeam, but no fewer, for launches of more regions
+ *                      than that or six 1024-sample chunks for each;
  *                      at most the workgroups that fit at once)
  *   balance            a team gets one workgroup per
  *                      total samples / (grid * balance) of its region (with

@@ -19,8 +19,9 @@ namespace pglgpu {
 // chunks per workgroup of the default grid from which a launch is bound by throughput
 static const uint64_t kManyChunks = 6;
 // workgroups that a launch bound by throughput leaves to another field's launch
-// beside it: the largest team of the default schedule, so that such a team is
-// always resident as a whole and none waits for the end of this launch
+// beside it, at the least: the largest team of the default schedule.  A schedule
+// with larger teams leaves as many as its largest, so that such a team is always
+// resident as a whole and none waits for the end of this launch
 static const uint32_t kLeaveGroups = 64;
 
 static void grow_pinned(void*& p, size_t& have, size_t need) {
@@ -135,12 +136,15 @@ void RegionRunner::stage(std::vector<RegionWork> work, const RegionSamplesView& 
     // the launch is bound by throughput and takes most of the device: 1029 and
     // 1957 regions of 700 samples 1.73 -> 1.58 and 0.73 -> 0.64 ms, 8 M samples
     // in 363 regions 7.1 -> 4.9 ms (1 M samples in 48 to 150 regions: 0 to 5 %
-    // slower).  With many chunks per workgroup teams twice as large shorten the
+    // slower).  Query server requests beside such launches wait as long as beside
+    // two per CU: requests of 4096 queries beside updates of 700k samples in 2514
+    // regions and of 10 M in 844, p99 0.23 and 0.10 ms (two per CU 0.24 and 0.09);
+    // of 65536 queries 0.47 and 0.35 ms (0.46 and 0.30).  With many chunks per workgroup teams twice as large shorten the
     // longest region, whose EM iterations are not known beforehand (10 M
     // samples in two fields, two frames: 16.6 -> 15.7 ms; at two chunks per
     // workgroup the smaller shares cost more than they give, 3.8 -> 4.0 ms).
-    if (work.size() > defaultGrid_ || chunks > kManyChunks * defaultGrid_)
-      G = std::max(defaultGrid_, resident_ - std::min(resident_, kLeaveGroups));
+    const uint32_t leave = std::min(resident_, std::max(kLeaveGroups, schedule.maxTeam));
+    if (work.size() > defaultGrid_ || chunks > kManyChunks * defaultGrid_) G = std::max(defaultGrid_, resident_ - leave);
     if (chunks > kManyChunks * defaultGrid_) bal *= 2.0;
   }
   const double target = std::max(total / ((double)G * bal), 1e-30);

@@ -82,3 +82,16 @@ def test_default_grid_rule(counts):
     chunks than it takes at once, against a small fixed grid"""
     recs, c, stats, init_k = _regions(counts, [(8, 16, 32)[r % 3] for r in range(len(counts))], seed=3)
     assert _state(_run(recs, c, stats, init_k)) == _state(_run(recs, c, stats, init_k, grid=96))
+
+
+@pytest.mark.parametrize("max_team", [16, 64, 65, 128, 200, 256, 1000])
+def test_default_grid_leaves_the_largest_team(max_team):
+    """a launch of more regions than the default grid takes leaves as many of the
+    resident workgroups as its largest team has, 64 at the least, down to the
+    default grid (two of three workgroups of a compute unit)"""
+    recs, c, stats, init_k = _regions([96] * 800, [8] * 800, seed=5)
+    resident = _run(recs, c, stats, init_k, grid=1 << 20).last_info()["grid"]
+    few = _run(recs[:96 * 500], c[:500], stats[:500], init_k[:500]).last_info()["grid"]
+    assert few == 500  # no more workgroups than items
+    batch = _run(recs, c, stats, init_k, max_team=max_team)
+    assert batch.last_info()["grid"] == max(resident * 2 // 3, resident - max(64, max_team))
