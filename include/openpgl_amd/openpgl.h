@@ -350,6 +350,10 @@ void pglFieldGetLastUpdateInfo(PGLField field, int kind, double* out, size_t cou
  * the field fails (prints the error, returns false / 0 / nothing) until
  * pglFieldReset. */
 void pglFieldDebugFailNextUpdate(PGLField field, int kind);
+/* EXTENSION (testing): the next pglFieldUpdateFromPathSegmentsDevice runs as if
+ * outputs with room for every vertex could not be allocated: the records are
+ * counted first, and the results are the same. */
+void pglFieldDebugFailNextPathOutputs(PGLField field);
 /* EXTENSION: the same figures for the last min(maxEntries, 256) updates of
  * one kind, oldest first, 19 doubles each ([13] is 0); returns the count.
  * Updates are queued (pglFieldUpdate* returns once the directional phase is

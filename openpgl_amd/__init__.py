@@ -121,6 +121,7 @@ _SIGS = {
     "pglFieldStatisticsToCSVString": (PGLString, [_vp]),
     "pglFieldStatisticsGetValues": (None, [_vp, _vp, ctypes.c_size_t]),
     "pglFieldDebugFailNextUpdate": (None, [_vp, ctypes.c_int]),
+    "pglFieldDebugFailNextPathOutputs": (None, [_vp]),
     "pglFieldArgumentsSetDefaults": (None, [ctypes.POINTER(PGLFieldArguments), ctypes.c_int, ctypes.c_int,
                                             ctypes.c_bool, ctypes.c_size_t]),
     "pglNewDevice": (_vp, [ctypes.c_int, ctypes.c_size_t]),
@@ -586,6 +587,10 @@ class Field:
     def debug_fail_next_update(self, kind=0):
         """pglFieldDebugFailNextUpdate (testing)."""
         self.lib.pglFieldDebugFailNextUpdate(self.h, kind)
+
+    def debug_fail_next_path_outputs(self):
+        """pglFieldDebugFailNextPathOutputs (testing)."""
+        self.lib.pglFieldDebugFailNextPathOutputs(self.h)
 
     def set_region_schedule(self, per_region_launches=None, grid=None, balance=None, min_chunks_per_rank=None,
                             max_team=None, cooperative=None):

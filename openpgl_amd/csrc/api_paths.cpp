@@ -311,4 +311,11 @@ void pglFieldUpdateFromPathSegmentsDevice(PGLField field, const PGLPathSegmentDa
 }
 PGL_CATCH_END_VOID
 
+void pglFieldDebugFailNextPathOutputs(PGLField field) PGL_CATCH_BEGIN {
+  THROW_IF_NULL(field, "handle");
+  if (!field->paths) field->paths = new PathSampleBatch();
+  field->paths->failNextFull = true;
+}
+PGL_CATCH_END_VOID
+
 }  // extern "C"

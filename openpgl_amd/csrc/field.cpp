@@ -147,6 +147,23 @@ void DevBuf::ensure(size_t b, bool keep) {
   p = np;
   bytes = nb;
 }
+bool DevBuf::tryEnsure(size_t b) {
+  if (b <= bytes) return true;
+  for (const size_t nb : {std::max(std::max(b, bytes * 2), size_t(65536)), b}) {
+    void* np = nullptr;
+    const hipError_t e = hipMalloc(&np, nb);
+    if (e == hipErrorOutOfMemory) {
+      (void)hipGetLastError();  // not for a later check
+      continue;
+    }
+    PGL_HIP_CHECK(e);
+    release();
+    p = np;
+    bytes = nb;
+    return true;
+  }
+  return false;
+}
 void DevBuf::release() {
   if (p) (void)hipFree(p);
   p = nullptr;

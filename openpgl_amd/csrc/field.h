@@ -71,6 +71,7 @@ struct DevBuf {
   void* p = nullptr;
   size_t bytes = 0;
   void ensure(size_t b, bool keep = false);
+  bool tryEnsure(size_t b);  // false, and as it was, where memory does not suffice
   void release();
   ~DevBuf() { release(); }
   template <class T> T* as() const { return (T*)p; }

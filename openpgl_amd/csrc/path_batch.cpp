@@ -104,8 +104,8 @@ void PathSampleBatch::prepareOwned(const PathVertex* segs, uint32_t numSegments,
                                    uint32_t numPaths, const PathSampleOptions& o, const PathSample*& surf,
                                    size_t& numSurf, const PathSample*& vol, size_t& numVol) {
   const int b = next_;
-  if (numSegments <= kFusedPathVertices) {
-    acquireOwned(b, numPaths ? numSegments : 0, numPaths ? numSegments : 0);
+  const size_t room = numPaths ? numSegments : 0;
+  if (numSegments <= kFusedPathVertices && acquireOwned(b, room, room, true)) {
     fused(segs, numSegments, offsets, numPaths, o, out_[b][0].as<PathSample>(), out_[b][1].as<PathSample>(), numSurf,
           numVol);
   } else {
@@ -123,7 +123,7 @@ void PathSampleBatch::prepareOwned(const PathVertex* segs, uint32_t numSegments,
   lastBuffer_ = b;
 }
 
-void PathSampleBatch::acquireOwned(int b, size_t numSurf, size_t numVol) {
+bool PathSampleBatch::acquireOwned(int b, size_t numSurf, size_t numVol, bool optional) {
   // the buffer's previous consumers (the gathers of an earlier update) must be done with it
   for (int k = 0; k < 2; k++)
     if (pendingRelease_[b][k]) {
@@ -131,10 +131,20 @@ void PathSampleBatch::acquireOwned(int b, size_t numSurf, size_t numVol) {
       pendingRelease_[b][k] = false;
     }
   const size_t ns = std::max<size_t>(numSurf, 1), nv = std::max<size_t>(numVol, 1);
-  if (out_[b][0].bytes < ns * sizeof(PathSample) || out_[b][1].bytes < nv * sizeof(PathSample))
+  const bool refuse = optional && failNextFull;
+  if (optional) failNextFull = false;
+  if (refuse || out_[b][0].bytes < ns * sizeof(PathSample) || out_[b][1].bytes < nv * sizeof(PathSample))
     PGL_HIP_CHECK(hipStreamSynchronize(stream_));  // a reallocation frees memory the wait above protects
-  out_[b][0].ensure(ns * sizeof(PathSample));
-  out_[b][1].ensure(nv * sizeof(PathSample));
+  if (!optional) {
+    out_[b][0].ensure(ns * sizeof(PathSample));
+    out_[b][1].ensure(nv * sizeof(PathSample));
+    return true;
+  }
+  if (!refuse && out_[b][0].tryEnsure(ns * sizeof(PathSample)) && out_[b][1].tryEnsure(nv * sizeof(PathSample)))
+    return true;
+  out_[b][0].release();
+  out_[b][1].release();
+  return false;
 }
 
 void PathSampleBatch::routeOwned(const PathSample* recs, uint32_t n, const PathSample*& surf, size_t& numSurf,

@@ -29,7 +29,9 @@ class PathSampleBatch {
   // Samples of the paths written into the batch's own double-buffered output
   // (for a field update that reads them after this call returns).  Before a
   // buffer is reused, the stream waits for `released` events recorded by
-  // the previous consumer of that buffer.
+  // the previous consumer of that buffer.  The outputs have room for every
+  // vertex (4 x 40 bytes per vertex, kept) where that can be allocated, and for
+  // the counted records elsewhere.
   void prepareOwned(const PathVertex* segs, uint32_t numSegments, const uint32_t* offsets, uint32_t numPaths,
                     const PathSampleOptions& o, const PathSample*& surf, size_t& numSurf, const PathSample*& vol,
                     size_t& numVol);
@@ -40,6 +42,9 @@ class PathSampleBatch {
                   const PathSample*& vol, size_t& numVol);
   // events after which the buffer handed out by the last prepareOwned / routeOwned may be overwritten
   void setReleased(hipEvent_t surfaceDone, hipEvent_t volumeDone);
+
+  // testing: the next outputs with room for every vertex cannot be allocated
+  bool failNextFull = false;
 
   hipStream_t stream() const { return stream_; }
 
@@ -55,8 +60,9 @@ class PathSampleBatch {
   // where the paths need them; blocks
   void fused(const PathVertex* segs, uint32_t numSegments, const uint32_t* offsets, uint32_t numPaths,
              const PathSampleOptions& o, PathSample* surfOut, PathSample* volOut, size_t& numSurf, size_t& numVol);
-  // output buffer b for ns / nv records, once its previous consumers are done
-  void acquireOwned(int b, size_t numSurf, size_t numVol);
+  // output buffer b for ns / nv records, once its previous consumers are done;
+  // optional: false, and the buffer given back, where memory does not suffice
+  bool acquireOwned(int b, size_t numSurf, size_t numVol, bool optional = false);
 
   hipStream_t stream_ = nullptr;
   DevBuf records_, flags_, pathOf_, tiles_, incl_, scanTemp_, totals_;

@@ -147,6 +147,26 @@ def test_field_update_with_and_without_long_paths(lengths):
     assert a.compare(b)
 
 
+def test_field_update_without_room_for_every_vertex():
+    """Where outputs for every vertex cannot be allocated, the records are counted
+    first: same states, whichever frames it happens in (the failure is set from
+    the host, nothing runs out of memory)."""
+    import openpgl_amd as pgl
+    from openpgl_amd.hip_runtime import DeviceArray
+    dev = pgl.Device()
+    a, b = pgl.Field(dev, max_samples_per_leaf=2000), pgl.Field(dev, max_samples_per_leaf=2000)
+    for frame, fail in enumerate((True, False, True, True, False)):
+        seg, off = random_paths(10000 + 3000 * frame, seed=300 + frame, max_len=8)
+        print("frame", frame, "vertices", len(seg), "no room" if fail else "", flush=True)
+        dseg, doff = DeviceArray.from_numpy(seg), DeviceArray.from_numpy(off)
+        for f in (a, b):
+            if fail and f is a:
+                f.debug_fail_next_path_outputs()
+            f.update_from_path_segments_device(dseg.value, len(seg), doff.value, len(off) - 1)
+        assert a.iteration() == b.iteration() == frame + 1
+        assert a.validate() and a.compare(b)
+
+
 _SHAPES = {
     "one vertex": ([1], 0, 0),
     "two vertices": ([2], 0, 0),
