@@ -371,8 +371,9 @@ size_t pglFieldGetUpdateHistory(PGLField field, int kind, double* out, size_t ma
  *   grid               workgroups of the persistent launch (0: two per CU,
  *                      which leaves room for other streams' kernels, and
  *                      the three that fit less the larger of 64 and
- *                      maxTeam, but no fewer, for launches of more regions
- *                      than that or six 1024-sample chunks for each;
+ *                      maxTeam, but no fewer, for launches of more than
+ *                      6144 samples for each of those, and for first fits
+ *                      and batches of more regions than those;
  *                      at most the workgroups that fit at once)
  *   balance            a team gets one workgroup per
  *                      total samples / (grid * balance) of its region (with

@@ -122,30 +122,38 @@ void RegionRunner::stage(std::vector<RegionWork> work, const RegionSamplesView& 
   const bool perRegion = schedule.perRegionLaunches != 0;
   const bool perRegionTeams = schedule.perRegionLaunches == 2;
   double total = 0.0;
-  uint64_t chunks = 0;
+  uint64_t samples = 0;
   for (const auto& w : work) {
     total += std::max(w.cost, 0.f);
-    chunks += std::max<uint32_t>(1, (w.samples + kChunk - 1) / kChunk);
+    samples += w.samples;
   }
   uint32_t G = perRegion ? 1u : (schedule.grid ? std::min(schedule.grid, resident_) : defaultGrid_);
   double bal = schedule.balance > 0.f ? schedule.balance : 1.f;
   if (!perRegion && schedule.grid == 0) {
     // The default grid leaves a third of the device to other streams' kernels
     // (the next update's spatial phase).  That pays while the launch is one
-    // wave of teams; with more regions than workgroups, or many chunks for each,
-    // the launch is bound by throughput and takes most of the device: 1029 and
-    // 1957 regions of 700 samples 1.73 -> 1.58 and 0.73 -> 0.64 ms, 8 M samples
-    // in 363 regions 7.1 -> 4.9 ms (1 M samples in 48 to 150 regions: 0 to 5 %
-    // slower).  Query server requests beside such launches wait as long as beside
-    // two per CU: requests of 4096 queries beside updates of 700k samples in 2514
-    // regions and of 10 M in 844, p99 0.23 and 0.10 ms (two per CU 0.24 and 0.09);
-    // of 65536 queries 0.47 and 0.35 ms (0.46 and 0.30).  With many chunks per workgroup teams twice as large shorten the
-    // longest region, whose EM iterations are not known beforehand (10 M
-    // samples in two fields, two frames: 16.6 -> 15.7 ms; at two chunks per
-    // workgroup the smaller shares cost more than they give, 3.8 -> 4.0 ms).
-    const uint32_t leave = std::min(resident_, std::max(kLeaveGroups, schedule.maxTeam));
-    if (work.size() > defaultGrid_ || chunks > kManyChunks * defaultGrid_) G = std::max(defaultGrid_, resident_ - leave);
-    if (chunks > kManyChunks * defaultGrid_) bal *= 2.0;
+    // wave of teams.  With many chunks for each workgroup it is bound by
+    // throughput and takes most of the device, and teams twice as large shorten
+    // its longest region, whose EM iterations are not known beforehand: queued
+    // updates of 4 M samples in 1119 regions 2.2 -> 1.9 ms, of 10 M in 1809
+    // regions 5.3 -> 4.7 ms, the first of them 14.2 -> 11.2 ms.
+    // With more regions than workgroups, first fits take it too (the first
+    // 700k samples in 2514 regions 2.3 -> 2.1 ms), and a batch of regions, beside
+    // which nothing is queued.  Later updates of many regions last no longer
+    // than the spatial phase beside them, which the larger grid slows down: 40
+    // queued updates of 1 M samples in 306 to 1429 regions 0.75 instead of 0.67
+    // ms each, in 3231 regions 1.02 instead of 0.99, 700k samples in 7738 regions
+    // 1.95 instead of 1.88; one such update with nothing behind it would gain 4 %.
+    // Query server requests beside updates of 10 M samples in 844 regions wait
+    // as long as beside two workgroups per CU: requests of 4096 queries p99 0.10
+    // ms (0.09), of 65536 queries 0.35 (0.30).
+    const bool chunks = samples > uint64_t(kChunk) * kManyChunks * defaultGrid_;
+    const bool fits = inputs == nullptr || (numInputs && inputs[0].mode == 1);  // every region's mode is the same
+    if (chunks || (fits && work.size() > defaultGrid_)) {
+      const uint32_t leave = std::min(resident_, std::max(kLeaveGroups, schedule.maxTeam));
+      G = std::max(defaultGrid_, resident_ - leave);
+    }
+    if (chunks) bal *= 2.0;
   }
   const double target = std::max(total / ((double)G * bal), 1e-30);
   const uint32_t minChunks = std::max<uint32_t>(1, schedule.minChunksPerRank);

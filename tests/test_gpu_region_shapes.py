@@ -85,13 +85,31 @@ def test_default_grid_rule(counts):
 
 
 @pytest.mark.parametrize("max_team", [16, 64, 65, 128, 200, 256, 1000])
-def test_default_grid_leaves_the_largest_team(max_team):
-    """a launch of more regions than the default grid takes leaves as many of the
-    resident workgroups as its largest team has, 64 at the least, down to the
-    default grid (two of three workgroups of a compute unit)"""
-    recs, c, stats, init_k = _regions([96] * 800, [8] * 800, seed=5)
-    resident = _run(recs, c, stats, init_k, grid=1 << 20).last_info()["grid"]
-    few = _run(recs[:96 * 500], c[:500], stats[:500], init_k[:500]).last_info()["grid"]
-    assert few == 500  # no more workgroups than items
-    batch = _run(recs, c, stats, init_k, max_team=max_team)
+@pytest.mark.parametrize("regions,samples", [(800, 96), (400, 8200)])
+def test_default_grid_leaves_the_largest_team(max_team, regions, samples):
+    """a batch of more regions, or more samples, than the default grid takes
+    leaves as many of the resident workgroups as its largest team has, 64 at the
+    least, down to the default grid (two of three workgroups of a compute unit)"""
+    resident = _run(*_regions([96] * 800, [8] * 800, seed=5), grid=1 << 20).last_info()["grid"]
+    batch = _run(*_regions([samples] * regions, [8] * regions, seed=5), max_team=max_team)
     assert batch.last_info()["grid"] == max(resident * 2 // 3, resident - max(64, max_team))
+
+
+def test_default_grid_of_updates():
+    """Updates of a field keep to the default grid, however many regions there
+    are, and take the larger one for a first fit of many regions or for many
+    samples."""
+    import openpgl_amd as pgl
+    from openpgl_amd.synth import generate
+    f = pgl.Field(pgl.Device(), max_samples_per_leaf=200, deterministic=True)
+    grids = []
+    for frame in range(3):
+        print("frame", frame, flush=True)
+        f.update(pgl.SampleStorage(generate(200000, seed=1, frame=frame)))
+        assert f.num_regions(0) > 1000
+        grids.append(f.last_update_info()["grid"])
+    resident = grids[0] + 64
+    assert resident % 3 == 0 and grids[1:] == [resident * 2 // 3] * 2
+    f = pgl.Field(pgl.Device(), deterministic=True)
+    f.update(pgl.SampleStorage(np.tile(generate(200000, seed=1), 17)))
+    assert f.num_regions(0) < 1000 and f.last_update_info()["grid"] == grids[0]
