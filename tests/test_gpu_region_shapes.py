@@ -1,7 +1,7 @@
 """The region kernel at the edges of its loops: sample counts around a wave, a
 workgroup and a chunk, component counts of every number of groups, directions
-that leave the range the bounded exponent assumes, and launches on either side
-of the default grid's rule.
+on both sides of the length from which the exponent itself is bounded, and
+launches on either side of the default grid's rule.
 
 Against the oracle (as the batched launch, tests/parity_checks.py) and bit for
 bit between schedules: how a region's samples are shared out changes no result.
@@ -36,10 +36,10 @@ def _regions(counts, ks, seed):
     return recs, np.asarray(counts, np.uint32), stats, np.asarray(ks, np.uint32)
 
 
-def _run(recs, counts, stats, init_k, **schedule):
+def _run(recs, counts, stats, init_k, deterministic=True, **schedule):
     import openpgl_amd as pgl
     from openpgl_amd.hip_runtime import DeviceArray
-    batch = pgl.RegionBatch(pgl.Device(), max_samples_per_leaf=32000)
+    batch = pgl.RegionBatch(pgl.Device(), max_samples_per_leaf=32000, deterministic=deterministic)
     if schedule:
         batch.set_schedule(**schedule)
     print("regions", len(counts), "samples", len(recs), "schedule", schedule, flush=True)
@@ -60,19 +60,46 @@ def test_sample_counts_and_groups(k):
     assert _state(batch) == _state(_run(recs, counts, stats, init_k, per_region_launches=0, balance=8.0, max_team=64))
 
 
-@pytest.mark.parametrize("scale", [1.5, 30.0])
-def test_directions_out_of_range(scale):
-    """a region with directions longer than one takes the loops that bound no
-    exponent: the same bits alone and in teams, its neighbours' bits unchanged"""
-    counts, ks = [300, 5000, 300], [8, 20, 32]
-    recs, c, stats, init_k = _regions(counts, ks, seed=7)
-    plain = _state(_run(recs, c, stats, init_k))
+def _odd_directions(scale, weight):
+    """three regions; some samples of the middle one, in the second and fourth of
+    its five chunks, have directions `scale` times a unit vector (at infinite
+    distance, so that the reprojection keeps them)"""
+    recs, c, stats, init_k = _regions([300, 5000, 300], [8, 20, 32], seed=7)
     recs = recs.copy()
-    recs["dir"][300 + 17:300 + 5000:100] *= np.float32(scale)
-    ref = _state(_run(recs, c, stats, init_k, per_region_launches=1))
+    odd = 300 + np.array([1024 + 5, 1024 + 77, 3072 + 900, 3072 + 901, 3072 + 1023])
+    recs["dir"][odd] *= np.float32(scale)
+    recs["distance"][odd] = np.inf
+    if weight is not None:
+        recs["weight"][odd] = weight
+    return recs, c, stats, init_k
+
+
+@pytest.mark.parametrize("weight", [None, 0.0])
+@pytest.mark.parametrize("scale", [1.5, 30.0, 1e13, 1e30, np.inf, np.nan])
+def test_directions_out_of_range(scale, weight):
+    """directions longer than one, on either side of the length from which a
+    chunk takes the loops that bound the exponent itself: the same bits alone and
+    in teams, the neighbours' bits unchanged"""
+    plain = _state(_run(*_odd_directions(1.0, weight), deterministic=False))
+    args = _odd_directions(scale, weight)
+    ref = _state(_run(*args, deterministic=False, per_region_launches=1))
     assert ref[0] == plain[0] and ref[2] == plain[2]
-    assert ref == _state(_run(recs, c, stats, init_k))
-    assert ref == _state(_run(recs, c, stats, init_k, per_region_launches=0, balance=8.0, max_team=64))
+    assert ref == _state(_run(*args, deterministic=False))
+    assert ref == _state(_run(*args, deterministic=False, per_region_launches=0, balance=8.0, max_team=64))
+
+
+def test_bounded_loops_equal_ordinary_ones():
+    """Directions 1e11 times a unit vector take the ordinary loops and 1e13 times
+    one the bounded loops, for every sample of their chunks; with weight 0 those
+    samples count alike, as every lobe is saturated at both lengths, so the
+    regions have the same bits, and finite ones."""
+    for schedule in (dict(per_region_launches=1), dict(), dict(per_region_launches=0, balance=8.0, max_team=64)):
+        a, b = (_run(*_odd_directions(scale, 0.0), deterministic=False, **schedule) for scale in (1e11, 1e13))
+        assert _state(a) == _state(b)
+        r = b.region(1)
+        assert r["valid"] and r["K"] > 4
+        for key in ("weights", "kappas", "meanDirections", "distances", "sumOfWeightedStats", "chiSquareMCEstimates"):
+            assert np.all(np.isfinite(np.asarray(r[key]))), key
 
 
 @pytest.mark.parametrize("counts", [[96 + r % 5 for r in range(511)], [96 + r % 5 for r in range(700)],
