@@ -345,7 +345,7 @@ void pglFieldGetKNN(PGLField field, int kind, uint32_t* neighbours /* 8 per regi
 void pglFieldGetLastUpdateInfo(PGLField field, int kind, double* out, size_t count);
 /* EXTENSION (testing): the next update of the field kind (0 surface, 1 volume)
  * is reported as failed once its kernels have run, as a region kernel whose
- * team barrier timed out is.  A failed update is reported by the call that
+ * wait for team partials timed out is.  A failed update is reported by the call that
  * completes it; from then on every update, query, export and file write of
  * the field fails (prints the error, returns false / 0 / nothing) until
  * pglFieldReset. */
@@ -398,7 +398,7 @@ typedef struct {
 void pglFieldSetRegionSchedule(PGLField field, const PGLRegionSchedule* schedule);
 /* EXTENSION: per-region profile of the last update, 12 floats per region in
  * storage order: microseconds of [0] the whole region, [1] E-step passes,
- * [2] split-statistics passes, [3] distance passes, [4] team barrier waits,
+ * [2] split-statistics passes, [3] distance passes, [4] waits for team partials,
  * [5] merging, [6] splitting logic, [9] M-steps and convergence tests,
  * [10] cross-chunk folds; [7] team size, [8] E-step passes, [11] samples. */
 void pglFieldGetRegionProfile(PGLField field, int kind, float* out);

@@ -618,7 +618,7 @@ class Field:
         return [dict(zip(_INFO_KEYS, o[i].tolist())) for i in range(n)]
 
     def region_profile(self, kind=0):
-        """(regions, 12): us of total, E-step, split, distance passes, barrier waits, merging,
+        """(regions, 12): us of total, E-step, split, distance passes, waits for team partials, merging,
         splitting logic, [7] team size, [8] E-step passes, [9] M-steps, [10] folds, [11] samples.
         Storage order."""
         out = np.zeros((self.num_regions(kind), 12), np.float32)

@@ -136,8 +136,8 @@ struct RegionState {
   // counts: [7] team size, [8] E-step passes, [11] samples
   float prof[12];
   int32_t initK;        // components of the initial mixture of a fit (0: the factory's initK)
-  // the mixture as the query kernel reads it, component by component: a quad
-  // of lanes reads four components' halves as one 64-byte line
+  // the mixture as the query kernel reads it, component by component: a lane
+  // reads a component as two 16-byte halves, a quad four components side by side
   struct alignas(16) QueryComp {
     float mux, muy, muz, dist, w, kappa, norm, unused;
   } query[32];

@@ -59,9 +59,13 @@
 #define PGL_REGION_KERNEL k_region_update
 // The split statistics pass uses all 168 VGPRs; called as a function it
 // saves the 33 callee-saved registers among them to scratch per lane on every
-// call, inlined into the update path it spills nothing.  (The EM loop, which
-// saves 47, runs slower inlined and stays a call.)  The fit path (first update
-// of a region) keeps its calls.
+// call, so it is inlined into the update path.  (The EM loop, which saves 47,
+// runs slower inlined and stays a call.)  The fit path (first update of a
+// region) keeps its calls.  With a loop for every group count and the bounded
+// one in each of the three passes the build spills all the same: 67 registers,
+// 808 bytes of scratch per lane (1 and 516 with loops for even counts of
+// groups and per-lane sums), 332 MB of HBM traffic for a launch of 1 M samples
+// in 50 to 275 regions (182 MB), 0.9 TB/s, which does not bound it.
 #define PGL_REGION_CALL __forceinline__
 #else
 #define PGL_REGION_KERNEL k_region_update_wide
@@ -2019,11 +2023,12 @@ __device__ void region_job(Shared& sh, Team& tm, RegionState* __restrict__ state
 // and every wait ends (given T <= grid, which the host guarantees, and a
 // grid that fits the device).  This file is compiled twice (each build with
 // its own device functions): PGL_REGION_OCC = 3 fits three workgroups on a CU
-// (168 VGPRs) and serves the default launch of two per CU, which leaves the
-// room of the third to other streams' kernels (the next update's spatial
-// phase); PGL_REGION_OCC = 2 (248 VGPRs, the faster code, k_region_update_wide)
-// serves launches of at most one workgroup per CU, which leave half of every
-// CU to other work (serving next to training).
+// (168 VGPRs, 808 bytes of scratch per lane) and serves the default launches,
+// most of them two per CU, which leaves the room of the third to other streams'
+// kernels (the next update's spatial phase); PGL_REGION_OCC = 2 (254 VGPRs, 520
+// bytes, the faster code, k_region_update_wide) serves launches of at most one
+// workgroup per CU, which leave half of every CU to other work (serving next to
+// training).
 __global__ void __launch_bounds__(RT) __attribute__((amdgpu_waves_per_eu(PGL_REGION_OCC, PGL_REGION_OCC)))
 PGL_REGION_KERNEL(RegionState* __restrict__ states,
                                                       const RegionJob* __restrict__ jobs,
